@@ -6,760 +6,643 @@
 // A 656-byte row holds 512 fp8 e4m3 "nope" features, 64 bf16 rope features and four fp32
 // scales (one per 128 nope features). key = [nope * scale, rope] (576 features), value =
 // nope * scale (512). For query row r and head h:
-//   out[r, h] = sum_j bf16(p_j) value_j / sum_j p_j,  p_j = exp(s_j - max_j s_j),
-//   s_j = scale * <q[r, h], key_j>  over the row's indices j >= 0,
-// i.e. softmax attention with bf16 probabilities in the value product (the reference rounds
-// the normalised probabilities to bf16; here the unnormalised ones, divided once at the end).
+//   out[r, h] = sum_j p_j value_j / sum_j p_j,  p_j = exp(s_j - max_j s_j),
+//   s_j = scale * <q[r, h], key_j>  over the row's indices j >= 0.
 //
-// Up to 32 heads, one workgroup per (query row, set of one or two groups of 16 heads, split
-// of the 2048 indices) resolves its indices to cache rows once (block table), then streams them
-// in tiles of 64 tokens: a tile's rows are gathered into registers two tiles ahead,
-// dequantised to bf16 with the hardware conversions (v_cvt_pk_f32_fp8, OCP e4m3 on gfx950,
-// and v_cvt_pk_bf16_f32) into one of two token-major LDS tile buffers once for every head
-// group of the set, the logits of the tile come from bf16 MFMA
-// (v_mfma_f32_16x16x32_bf16: 16 heads x 16 tokens x 32 features), an online softmax keeps the
-// running maximum and sum per head, and the value product is a second MFMA (16 heads x 16
-// features x 32 tokens) accumulated in registers, its value fragments (8 tokens of one
-// feature per lane) read from the same key tile by gfx950's transpose loads
-// (ds_read_b64_tr_b16); the next tile is staged beside it. Splits (up to 8, enough workgroups to fill
-// the chip) leave (max, sum, unnormalised output) per head in the workspace and a second
-// launch merges them. HBM traffic is one read of each selected row plus the partials.
-// More than 32 heads run on sparse_attention_pair_kernel (groups of four waves per 32 heads,
-// 32x32x16 MFMAs, described there), which leaves the same partial records.
-#include "kvip_device.h"
+// A workgroup takes (query row, set of one or two groups of 16 heads, split of the 2048 indices).
+// It resolves its indices to cache rows once (block table), then streams them as four token
+// streams of 32-token tiles, one wave per stream and head group. A wave keeps its group's query
+// and the whole [16 heads, 512] accumulator in registers and exchanges nothing until the four
+// streams' softmaxes are merged through LDS at the end; the waves of the two groups share the
+// tiles of a stream (one barrier per tile and one per rope buffer; a single group has none).
+//   - A tile stays as it is in the cache: direct-to-LDS loads put its 512 fp8 bytes per token into a
+//     two-slot ring, tile k + 4 landing while tile k is computed. No dequantised copy is made.
+//   - Logits: fp8 MFMA (16x16x128, one scale group per instruction) of the raw key bytes with the
+//     query as two fp8 terms, which hold bf16's eight significant bits, so no key byte is
+//     converted; each scale group's dot products are summed on their own and added as
+//     fma(group, scale, s) in fp32. The rope features are bf16 MFMA.
+//   - Values: bf16 MFMA of the value bytes, converted as they are read (two features per
+//     v_cvt_scalef32_pk_bf16_fp8 with scale 1, exact), with the probabilities times the group's
+//     scale (fp32, then rounded to bf16). One rounding per product instead of one on either side.
+//   - The logits are computed transposed (tokens as M, heads as N), so a lane holds one head's logits
+//     of 8 tokens: the softmax takes two lane swaps per tile, and the probabilities are the value
+//     product's B operand (features as M, heads as N) without leaving their registers, because
+//     the token order along K is free as long as both operands share it. The value operand (8
+//     tokens of one feature per lane) comes from the token-major tile by ds_read_b64_tr_b8, whose
+//     lanes address the tokens in that order.
+//   - The running maximum is rescaled lazily: only when a tile's maximum exceeds it by kSaMargin (the
+//     probabilities are then at most e^8, well inside bf16 and fp32), which after a row's first
+//     tiles is rare.
+//
+// What bounds it: 16 heads read each row once, ~5 TB/s of 128-byte lines, between ~6 us of start
+// (indices, table, first tile) and ~7 us of merges; more heads are bound by issue and LDS reads
+// (about 620 instructions per wave and tile). LDS (ring 128 KB, rope 16 KB, cache rows 8 KB,
+// scales 4 KB) allows one workgroup per CU. Measured, 64 rows, against the version that
+// dequantised tiles to bf16 in LDS and exchanged probabilities between waves: 16 heads of 16384
+// hot slots 37.6 -> 30.4 us per call, 128 heads of 2048 slots 98.8 -> 71.8; 32 heads 47.1 -> 34.4,
+// 64 heads 58.2 -> 45.4; one row of 16 heads 21.7 -> 13.0. Error against 64 bits on N(0, 1) rows:
+// 1.1e-3 (1.9e-3 with both sides rounded).
+// A variant with groups of 32 heads per wave (32x32x16 MFMA, 256 accumulators) spilled (356 us at 128
+// heads); scratch reloads wait for every load in flight, so the tile loop must not spill.
+#include "lds_async.h"
 
 namespace kvip {
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef int i32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kSaThreads = 256;
-constexpr int kSaTile = 64;                 // tokens per tile
-constexpr int kSaHeads = 16;                // heads per workgroup (MFMA M)
+constexpr int kSaHeads = 16;                // heads per wave (MFMA N)
+constexpr int kSaStreams = 4;               // token streams per workgroup
+constexpr int kSaTile = 32;                 // tokens per tile (value MFMA K)
 constexpr int kKeyDim = 576;                // 512 nope + 64 rope
 constexpr int kValueDim = 512;
-constexpr int kPieces = KVIP_KV_ROW_BYTES / 16;  // 41 pieces of a row, the last holds the scales
-constexpr int kPitch = kKeyDim + 8;         // bf16 per LDS key row (16 bytes of padding)
-constexpr int kPPitch = kSaTile + 8;        // bf16 per LDS probability row
-constexpr int kTokGroup = 8;  // tokens staged per thread
-constexpr int kPartial = 2 * kSaHeads + kSaHeads * kValueDim;  // floats per split: max, sum, output
-constexpr int kMaxSplits = 8;
+constexpr int kScaleGroups = 4;             // 128 nope features share a scale
+constexpr int kMaxSplits = 16;
+constexpr int kPartial = kValueDim + 2;     // floats per (row, head, split): output, max, sum
+constexpr float kLog2e = 1.44269504088896341f;
+constexpr float kSaMargin = 8.0f * kLog2e;  // lazy rescale: 8 in natural-log units
 
-// Index splits per (row, head-group set): doubled up to 8 while the launch has fewer than 256
-// workgroups (one per CU: the kernel holds one workgroup per CU).
-__host__ __device__ inline int sa_splits(int rows, int sets) {
-    int s = 1;
-    while (s < kMaxSplits && static_cast<int64_t>(rows) * sets * s < 256) s *= 2;
-    return s;
+// LDS map (bytes): per stream two tile slots of nope bytes, one tile of rope, two tiles of
+// scales [group][token]; the cache rows of the split's indices; per stream a tile's row addresses;
+// the query's block exponents and second rope fragments (two waves per SIMD leave 256 registers,
+// 128 of them accumulators).
+constexpr int kNopeSlot = kSaTile * kValueDim;
+constexpr int kRopeSlot = kSaTile * 128;
+constexpr int kScaleSlot = kScaleGroups * kSaTile * 4;
+constexpr int kLdsRope = kSaStreams * 2 * kNopeSlot;
+constexpr int kLdsScale = kLdsRope + kSaStreams * kRopeSlot;
+constexpr int kLdsRows = kLdsScale + kSaStreams * 2 * kScaleSlot;
+constexpr int kLdsBase = kLdsRows + kTopK * 4;
+constexpr int kLdsQuery = kLdsBase + kSaStreams * kSaTile * 8;  // query exponents, then a rope fragment per group
+constexpr int kLdsBytes = kLdsQuery + 2 * kSaHeads * kScaleGroups * 4 + 2 * 1024;
+static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
+
+// Head groups of 16 per workgroup, and workgroups per row before index splits.
+__host__ __device__ inline int sa_group_set(int heads) { return heads > kSaHeads ? 2 : 1; }
+__host__ __device__ inline int sa_sets(int heads) {
+    const int per = kSaHeads * sa_group_set(heads);
+    return (heads + per - 1) / per;
+}
+
+// Index splits per (row, head set): the count with the shortest estimated launch, in units of
+// one tile per stream (about 1 us): rounds of 256 workgroups (one per CU), each of its tiles per
+// stream plus about 3 for resolving the indices, the first tile's latency and the merge of the
+// streams; 5 more for the merge launch when there are splits.
+__host__ __device__ inline int sa_splits(int rows, int heads) {
+    const int64_t units = static_cast<int64_t>(rows) * sa_sets(heads);
+    int best = 1;
+    int64_t best_cost = 0;
+    for (int s = 1; s <= kMaxSplits; s *= 2) {
+        const int64_t cost = (units * s + 255) / 256 * (kTopK / (kSaTile * kSaStreams) / s + 3) + (s > 1 ? 5 : 0);
+        if (s == 1 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+typedef __attribute__((address_space(3))) const v4i* LdsV4i;
+typedef __attribute__((address_space(3))) const f32x4* LdsF32x4;
+typedef __attribute__((address_space(3))) i32x2* LdsI32x2;
+
+// x, recomputed from here on: keeps the compiler from hoisting the dozens of addresses derived
+// from a loop constant out of the tile loop, where they would not fit the registers.
+KVIP_DEVICE int fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
 }
 
 KVIP_DEVICE uint32_t pack_bf16(float a, float b) {  // hardware round to nearest even
     const bf16x2 v = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-    uint32_t u;
-    __builtin_memcpy(&u, &v, 4);
-    return u;
+    return __builtin_bit_cast(uint32_t, v);
 }
 
-KVIP_DEVICE uint16_t bf16_bits(float f) {  // round to nearest even (finite inputs)
-    uint32_t u = __float_as_uint(f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return static_cast<uint16_t>(u >> 16);
+// Eight fp8 e4m3 features as bf16 (exact).
+KVIP_DEVICE bf16x8 fp8x8_to_bf16(int lo, int hi) {
+    const v4i r = {
+        __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, false)),
+        __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.0f, true)),
+        __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false)),
+        __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true))};
+    return __builtin_bit_cast(bf16x8, r);
 }
 
-// Value of the lane chosen by a DPP control within each row of 16 lanes.
-template <int CTRL>
-KVIP_DEVICE float dpp(float x) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
+// Direct-to-LDS loads as inline asm: 16 (4) bytes per lane from src to lds + lane * 16 (4),
+// lds wave-uniform. LLVM waits for every pending load of the builtin form before each LDS read;
+// the asm form is waited for explicitly once per tile, and the LDS reads stay ordinary code. The
+// loads have no output registers, so nothing can be reused while they are in flight; no other
+// instruction of the kernel uses m0.
+KVIP_DEVICE void dma16(const uint8_t* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory");
 }
-// Max / sum over the 16 lanes of a row, in every lane of it: row mirror, half-row mirror,
-// then the two quad swaps; every lane's value enters each result exactly once.
-KVIP_DEVICE float row_max16(float x) {
-    x = fmaxf(x, dpp<0x140>(x));  // row_mirror
-    x = fmaxf(x, dpp<0x141>(x));  // row_half_mirror
-    x = fmaxf(x, dpp<0xB1>(x));   // quad_perm [1, 0, 3, 2]
-    return fmaxf(x, dpp<0x4E>(x));  // quad_perm [2, 3, 0, 1]
-}
-KVIP_DEVICE float row_sum16(float x) {
-    x += dpp<0x140>(x);
-    x += dpp<0x141>(x);
-    x += dpp<0xB1>(x);
-    return x + dpp<0x4E>(x);
+KVIP_DEVICE void dma4(const uint8_t* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory");
 }
 
-KVIP_DEVICE bf16x8 as_bf16x8(v4i v) {
-    bf16x8 r;
-    __builtin_memcpy(&r, &v, 16);
-    return r;
-}
-
-// Head groups of 16 handled by one workgroup: G share every staged tile (its gather and
-// dequantisation); group g runs on waves 4 g .. 4 g + 3, which keep its Q fragments,
-// online-softmax state and value accumulators in registers (G waves per SIMD).
-__host__ __device__ inline int sa_group_set(int heads) { return heads > kSaHeads ? 2 : 1; }
-// Workgroups per row before index splits: more than 32 heads run on
-// sparse_attention_pair_kernel, kPrGroups groups of 32 heads per workgroup, kPrSplit waves
-// per group.
-constexpr int kPrGroups = 2;
-constexpr int kPrSplit = 4;
-__host__ __device__ inline bool sa_pairs(int heads) { return heads > 2 * kSaHeads; }
-__host__ __device__ inline int sa_sets(int heads) {
-    if (sa_pairs(heads)) return ((heads + 31) / 32 + kPrGroups - 1) / kPrGroups;
-    const int groups = (heads + kSaHeads - 1) / kSaHeads;
-    return (groups + sa_group_set(heads) - 1) / sa_group_set(heads);
-}
-
-template <int G>
-__global__ __launch_bounds__(kSaThreads * G, 1) void sparse_attention_kernel(const KvipSparseAttnArgs p) {
-    constexpr int kThreads = kSaThreads * G;
-    constexpr int kFeat = 16 / G;  // nope features per thread and token (16-byte or 8-byte pieces)
-    __shared__ __align__(16) uint16_t s_k[2][kSaTile * kPitch];      // keys, token-major, two tiles
-    __shared__ __align__(16) uint16_t s_p[G][kSaHeads * kPPitch];
-    __shared__ float s_red[G][4][kSaHeads];
-    __shared__ int32_t s_row[kTopK];  // cache row (block * 128 + offset) of each index, -1 = none
-
-    // XCD-aware order: the workgroups of a query row (head-group sets x splits) share
-    // blockIdx % 8, so they run on one XCD, whose L2 then serves the row's KV rows and query to
-    // every set after the first read.
-    const int groups = (p.heads + kSaHeads - 1) / kSaHeads;
-    const int sets = (groups + G - 1) / G;
-    const int splits = sa_splits(p.rows, sets);
-    const int units = sets * splits;
-    const int chunk = blockIdx.x / (8 * units), within = blockIdx.x % (8 * units);
-    const int r = chunk * 8 + within % 8;
-    const int unit = within / 8, hs = unit % sets, sp = unit / sets;
-    if (r >= p.rows) return;
-    const int b = r / p.rows_per_request;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int gw = tid >> 8;           // head group of this wave within the set
-    const int w = (tid >> 6) & 3;      // quarter: logits of tokens 16 w .., values of features 128 w ..
-    const int lr = lane & 15, lg = lane >> 4;  // MFMA lane row / group
-    const int grp = hs * G + gw;
-    const bool live = grp < groups;    // uniform per wave: a set's last group may hold no heads
-    uint32_t err = 0;
-
-    // Cache rows of the split's indices, resolved once through the block table.
-    const int span = kTopK / splits;
-    const int* idx_row = p.indices + static_cast<size_t>(r) * kTopK + sp * span;
-    const int capacity = p.max_blocks * kBlockTokens;
-    for (int i = tid; i < span; i += kThreads) {
-        const int t = idx_row[i];
-        int row = -1;
-        if (t >= capacity) {
-            err |= KVIP_STATUS_BAD_TOKEN;
-        } else if (t >= 0) {
-            const int blk = p.block_table[static_cast<size_t>(b) * p.max_blocks + (t >> 7)];
-            if (static_cast<unsigned>(blk) < static_cast<unsigned>(p.num_blocks)) {
-                row = blk * kBlockTokens + (t & 127);
-            } else {
-                err |= KVIP_STATUS_BAD_BLOCK;
-            }
-        }
-        s_row[i] = row;
-    }
-
-    // Query fragments (A operand of the logits) of the wave's group: head 16 grp + lr,
-    // features 32 s + 8 lg .. + 8; heads past p.heads read as zero.
-    bf16x8 qf[kKeyDim / 32];
-    {
-        const int h = grp * kSaHeads + lr;
-        const bool hl = h < p.heads;
-        const uint16_t* q = p.query + (static_cast<size_t>(r) * p.heads + (hl ? h : 0)) * kKeyDim;
-#pragma unroll
-        for (int s = 0; s < kKeyDim / 32; ++s) {
-            const v4i v = hl ? *reinterpret_cast<const v4i*>(q + s * 32 + lg * 8) : v4i{0, 0, 0, 0};
-            qf[s] = as_bf16x8(v);
-        }
-    }
-    f32x4 acc[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_run[4], l_part[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        m_run[i] = -INFINITY;
-        l_part[i] = 0.f;
-    }
-    __syncthreads();
-
-    // Staging map: thread (token group tg, nope slice pc) holds kFeat nope features
-    // [16 pc' + kFeat h, + kFeat) of the 8 tokens 8 tg .. 8 tg + 7 (pc' = pc % 32, h = the
-    // thread's half of the piece when two workgroup halves share it), and the tile's 512
-    // rope pieces are dealt over every thread. Tile k + 2's pieces are requested right after
-    // tile k + 1 is staged (during tile k), so that their latency passes under a whole tile.
-    const int tg = (tid >> 5) & 7, pc = tid & 31, half = tid >> 8;
-    const int f0 = pc * 16 + half * kFeat;  // first nope feature of the thread
-    constexpr int kRope = kSaTile * 8 / kThreads;
-    typedef int vfi __attribute__((ext_vector_type(kFeat / 4)));
-    vfi nope[kTokGroup];
-    v4i rope[kRope];
-    float sc[kTokGroup];
-    auto row_base = [&](int row) {
-        return p.kv_cache + static_cast<int64_t>(row >> 7) * p.kv_block_stride +
-               static_cast<int64_t>(row & 127) * p.row_stride;
-    };
-    auto load_tile = [&](int k) {
-#pragma unroll
-        for (int u = 0; u < kTokGroup; ++u) {
-            const int row = s_row[k * kSaTile + tg * kTokGroup + u];
-            nope[u] = vfi{};
-            sc[u] = 0.f;
-            if (row >= 0) {
-                const uint8_t* base = row_base(row);
-                nope[u] = *reinterpret_cast<const vfi*>(base + f0);
-                sc[u] = *reinterpret_cast<const float*>(base + 640 + (pc >> 3) * 4);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kRope; ++j) {
-            const int q = j * kThreads + tid;
-            const int row = s_row[k * kSaTile + (q >> 3)];
-            rope[j] = row >= 0 ? *reinterpret_cast<const v4i*>(row_base(row) + 512 + (q & 7) * 16) : v4i{0, 0, 0, 0};
-        }
-    };
-    // Dequantisation to bf16: keys [nope * scale, rope] token-major into tile buffer kb. The
-    // values are the same nope * scale features, read feature-wise by the transpose loads.
-    auto stage_tile = [&](uint16_t* kb) {
-#pragma unroll
-        for (int u = 0; u < kTokGroup; ++u) {
-            uint32_t out[kFeat / 2];  // features f0 + 2k, 2k + 1
-#pragma unroll
-            for (int k = 0; k < kFeat / 4; ++k) {
-                const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(nope[u][k], false);
-                const f32x2 c = __builtin_amdgcn_cvt_pk_f32_fp8(nope[u][k], true);
-                out[2 * k] = pack_bf16(a[0] * sc[u], a[1] * sc[u]);
-                out[2 * k + 1] = pack_bf16(c[0] * sc[u], c[1] * sc[u]);
-            }
-            uint16_t* d = kb + (tg * kTokGroup + u) * kPitch + f0;
-            if constexpr (kFeat == 16) {
-                reinterpret_cast<v4i*>(d)[0] = v4i{static_cast<int>(out[0]), static_cast<int>(out[1]),
-                                                   static_cast<int>(out[2]), static_cast<int>(out[3])};
-                reinterpret_cast<v4i*>(d)[1] = v4i{static_cast<int>(out[4]), static_cast<int>(out[5]),
-                                                   static_cast<int>(out[6]), static_cast<int>(out[7])};
-            } else {
-                *reinterpret_cast<v4i*>(d) = v4i{static_cast<int>(out[0]), static_cast<int>(out[1]),
-                                                 static_cast<int>(out[2]), static_cast<int>(out[3])};
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < kRope; ++j) {
-            const int q = j * kThreads + tid;
-            *reinterpret_cast<v4i*>(kb + (q >> 3) * kPitch + 512 + (q & 7) * 8) = rope[j];
-        }
-    };
-    // Transpose-load address of this lane within a tile: in 16-lane block lg, lane lr reads 4
-    // features of one token and receives one feature (lr) of 4 consecutive tokens, i.e. block lg
-    // covers tokens 8 lg + 4 j .. + 4 (j = 0, 1: two loads) of 16 features: the B operand lane
-    // (feature lr, tokens 8 lg .. + 8) of the value MFMA.
-    const int tr_off = (8 * lg + (lr >> 2)) * kPitch + 4 * (lr & 3);
-
-    const int tiles = span / kSaTile;
-    load_tile(0);
-    stage_tile(s_k[0]);
-    if (tiles > 1) load_tile(1);
-    __syncthreads();  // s_k[0] holds tile 0
-    for (int k = 0; k < tiles; ++k) {
-        const uint16_t* kt = s_k[k & 1];
-        const bool more = k + 1 < tiles;
-        const bool tok_live = s_row[k * kSaTile + w * 16 + lr] >= 0;
-        // Logits of tokens 16 w .. 16 w + 15: lane holds heads 4 lg + i of token 16 w + lr.
-        float lg_v[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-        if (live) {
-            f32x4 sv = f32x4{0.f, 0.f, 0.f, 0.f};
-            const uint16_t* kr = kt + (w * 16 + lr) * kPitch + lg * 8;
-#pragma unroll
-            for (int s = 0; s < kKeyDim / 32; ++s) {
-                const bf16x8 kv = as_bf16x8(*reinterpret_cast<const v4i*>(kr + s * 32));
-                sv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf[s], kv, sv, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                lg_v[i] = tok_live ? sv[i] * p.scale : -INFINITY;
-                const float mx = row_max16(lg_v[i]);
-                if (lr == 0) s_red[gw][w][lg * 4 + i] = mx;
-            }
-        }
-        __syncthreads();
-        float alpha[4] = {1.f, 1.f, 1.f, 1.f};
-        if (live) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int h = lg * 4 + i;
-                const float tile_max =
-                    fmaxf(fmaxf(s_red[gw][0][h], s_red[gw][1][h]), fmaxf(s_red[gw][2][h], s_red[gw][3][h]));
-                const float m_new = fmaxf(m_run[i], tile_max);
-                alpha[i] = m_new == -INFINITY ? 1.f : __expf(m_run[i] - m_new);
-                m_run[i] = m_new;
-                const float pr = m_new == -INFINITY ? 0.f : __expf(lg_v[i] - m_new);
-                l_part[i] = l_part[i] * alpha[i] + pr;
-                s_p[gw][h * kPPitch + w * 16 + lr] = bf16_bits(pr);
-            }
-        }
-        __syncthreads();  // s_p complete; s_red free for the next tile
-        if (live) {
-            // Value product for features 128 w .. 128 w + 127 (8 MFMA columns of 16).
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[t][i] *= alpha[i];
-            }
-#pragma unroll
-            for (int ks = 0; ks < kSaTile / 32; ++ks) {
-                const bf16x8 pa = as_bf16x8(*reinterpret_cast<const v4i*>(&s_p[gw][lr * kPPitch + ks * 32 + lg * 8]));
-                // B fragment: tokens ks * 32 + 8 lg .. + 8 of feature 128 w + 16 t + lr.
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const uint16_t* vr = kt + tr_off + ks * 32 * kPitch + w * 128 + t * 16;
-                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(vr));
-                    const v4s hi =
-                        __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(vr + 4 * kPitch));
-                    const bf16x8 vb = __builtin_bit_cast(bf16x8, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vb, acc[t], 0, 0, 0);
-                }
-            }
-            // The next tile's staging beside this tile's value MFMAs, then the loads of the
-            // tile after it.
-            if (more) {
-                stage_tile(s_k[(k + 1) & 1]);
-                if (k + 2 < tiles) load_tile(k + 2);
-            }
-        } else if (more) {
-            stage_tile(s_k[(k + 1) & 1]);
-            if (k + 2 < tiles) load_tile(k + 2);
-        }
-        __syncthreads();  // tile k + 1 staged; tile k's buffer and s_p free
-    }
-
-    // Row sums: over the 16 lanes of a group, then over the group's waves; then this split's
-    // partial (max, sum, unnormalised output per head) or the normalised output.
-    float l_tot[4];
-    if (live) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float l = row_sum16(l_part[i]);
-            if (lr == 0) s_red[gw][w][lg * 4 + i] = l;
-        }
-    }
-    __syncthreads();
-    if (live) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int h = lg * 4 + i;
-            l_tot[i] = s_red[gw][0][h] + s_red[gw][1][h] + s_red[gw][2][h] + s_red[gw][3][h];
-        }
-        if (splits > 1) {
-            float* ws = p.workspace + ((static_cast<size_t>(r) * groups + grp) * splits + sp) * kPartial;
-            if (w == 0 && lr == 0) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    ws[lg * 4 + i] = m_run[i];
-                    ws[kSaHeads + lg * 4 + i] = l_tot[i];
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float* o = ws + 2 * kSaHeads + (lg * 4 + i) * kValueDim + w * 128 + lr;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) o[t * 16] = acc[t][i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int h = grp * kSaHeads + lg * 4 + i;
-                if (h >= p.heads) continue;
-                const float inv = l_tot[i] > 0.f ? 1.f / l_tot[i] : 0.f;
-                float* o = p.output + (static_cast<size_t>(r) * p.heads + h) * kValueDim + w * 128 + lr;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) o[t * 16] = acc[t][i] * inv;
-            }
-        }
-    }
-    report(p.status, err);
-}
-
-// More than 32 heads: groups of SPLIT = 4 waves per 32 heads. A workgroup (row, index split)
-// holds GROUPS such groups (GROUPS x 32 heads), so a staged tile of 32 rows serves all of
-// them once. Wave (th, hh) of a group computes the logits of the tile's tokens 16 th .. + 16
-// for heads 16 hh .. + 16 over all 576 features (v_mfma_f32_16x16x32_bf16, tokens as M, its 16
-// heads' query fragments as N), so no partial logits are exchanged and each logit is
-// exponentiated once: the two token halves exchange only their per-head maxima (LDS), every
-// wave of the group derives the same reference maxima for all 32 heads from them, and each
-// writes its 16 x 16 block of bf16 probabilities to LDS. For the value product each wave then
-// takes all 32 heads (v_mfma_f32_32x32x16_bf16, heads as M, probabilities read from LDS as the
-// A operand) and accumulates 512 / SPLIT of the value features (blocks of 32). The values are
-// the key tile's nope features: the value MFMA's B operand (8 tokens of one feature per lane)
-// comes from the token-major key tile by gfx950's transpose loads (ds_read_b64_tr_b16), so a
-// tile is dequantised and written to LDS once, and two tile buffers let the next tile be
-// staged beside this tile's value MFMAs (three barriers per tile). The running maximum is
-// rescaled lazily: only when a tile's maximum exceeds it by kPrMargin (the probabilities are
-// then at most e^kPrMargin, well inside bf16 and fp32), which after the first tiles of a row
-// is rare, so the 128 accumulators per lane are seldom touched outside the MFMAs.
-constexpr int kPrTile = 32;                  // tokens per tile
-constexpr int kPrKPitch = kKeyDim + 8;       // bf16 per K row: an odd number of 16-byte units
-constexpr int kPrPPitch = kPrTile + 8;       // bf16 per probability row
-typedef int i32x2 __attribute__((ext_vector_type(2)));
-constexpr float kPrLog2e = 1.44269504088896341f;
-constexpr float kPrMargin = 8.0f;            // natural-log units
-
-KVIP_DEVICE float lane_half_other(float x, int g) {  // x of lane l ^ 32
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
-    return __int_as_float(g == 0 ? sw[1] : sw[0]);
-}
-
-KVIP_DEVICE float rows4_max(float x) {  // max over lanes l, l ^ 16, l ^ 32, l ^ 48
+// Max / sum over lanes l, l ^ 16, l ^ 32, l ^ 48.
+KVIP_DEVICE float rows4_max(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-KVIP_DEVICE float rows4_sum(float x) {  // sum over lanes l, l ^ 16, l ^ 32, l ^ 48
+KVIP_DEVICE float rows4_sum(float x) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int GROUPS, int SPLIT>
-__global__ __launch_bounds__(GROUPS * SPLIT * 64, 1) void sparse_attention_pair_kernel(const KvipSparseAttnArgs p) {
-    static_assert(SPLIT == 4, "four waves per 32 heads");
-    constexpr int kThreads = GROUPS * SPLIT * 64;
-    constexpr int kKSteps = kKeyDim / 32;          // logit MFMA steps (16x16x32)
-    constexpr int kVPart = kValueDim / SPLIT;      // value features per wave
-    constexpr int kBlocks = kVPart / 32;           // value blocks of 32 features per wave
-    constexpr int kTokPer = kPrTile * 32 / kThreads;  // tokens each thread stages (2 or 4)
-    static_assert(kTokPer == 2 || kTokPer == 4, "staging map");
-    __shared__ __align__(16) uint16_t s_k[2][kPrTile * kPrKPitch];  // keys, token-major, two tiles
-    __shared__ __align__(16) uint16_t s_p[GROUPS][32 * kPrPPitch];  // probabilities, [head][token]
-    __shared__ float s_m[GROUPS][2][32];                             // per token half: head maxima / sums
-    __shared__ __align__(16) float s_h[GROUPS * SPLIT][32];          // per-head values for the O layout
-    __shared__ int32_t s_row[kTopK];
+// Places of a token's 16-byte pieces in its 512-byte LDS row: piece j sits at place j ^ swz(token).
+// Linear over XOR, and such that both a key read (16 consecutive lanes: one piece of 16 consecutive
+// tokens) and a value read (two 16-lane blocks of a transpose load: one piece of the 8 tokens
+// 4 kg .. + 3 and 16 + 4 kg .. + 3 for kg and kg + 1) touch every bank once.
+KVIP_DEVICE constexpr int sa_swz(int t) { return (t & 7) | ((((t >> 3) ^ (t >> 4)) & 1) << 3); }
 
-    const int pairs_needed = (p.heads + 31) / 32;
-    const int sets = (pairs_needed + GROUPS - 1) / GROUPS;
-    const int splits = sa_splits(p.rows, sets);
-    const int units = sets * splits;
-    // XCD-aware order as in the 16-head kernel: a row's workgroups share blockIdx % 8.
-    const int chunk = blockIdx.x / (8 * units), within = blockIdx.x % (8 * units);
-    const int r = chunk * 8 + within % 8;
-    const int unit = within / 8, hs = unit % sets, sp = unit / sets;
+// 16 tokens x 16 heads over 128 features: fp8 keys (scale 1) by fp8 query terms with block scale
+// byte g of `scales`.
+KVIP_DEVICE f32x4 sa_mma8(v8i a, v8i b, f32x4 c, int g, int scales) {
+    switch (g) {  // a constant after unrolling: the byte select is an immediate
+        case 0: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 0, scales);
+        case 1: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 1, scales);
+        case 2: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 2, scales);
+        default: return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 3, scales);
+    }
+}
+
+// Barrier for LDS data: unlike __syncthreads it leaves the direct-to-LDS loads in flight.
+KVIP_DEVICE void lds_sync() {
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" : : : "memory");
+}
+
+template <int G>
+__global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kernel(const KvipSparseAttnArgs p,
+                                                                                  int splits) {
+    constexpr int kWaves = kSaStreams * G;
+    constexpr int kThreads = kWaves * 64;
+    constexpr int kBlocks = kValueDim / 16;            // accumulator blocks of 16 features
+    __shared__ __align__(16) uint8_t s_mem[kLdsBytes];
+    int32_t* s_row = reinterpret_cast<int32_t*>(s_mem + kLdsRows);
+
+    // XCD-aware order: the head sets of one (query row, split), which read the same KV rows, share
+    // blockIdx % 8, so they run on one XCD, whose L2 then serves the rows to every set after the first
+    // read; rows and splits are dealt over all XCDs.
+    const int sets = sa_sets(p.heads);
+    const int chunk = blockIdx.x / (8 * sets), within = blockIdx.x % (8 * sets);
+    const int job = chunk * 8 + within % 8, hs = within / 8;
+    const int r = job / splits, sp = job % splits;
     if (r >= p.rows) return;
     const int b = r / p.rows_per_request;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int gi = w / SPLIT, hf = w % SPLIT;        // group in the workgroup, wave in the group
-    const int pair = hs * GROUPS + gi;               // 32-head group
-    const int th = hf & 1, hh = hf >> 1;             // logits of tokens 16 th .., heads 16 hh ..
-    const bool live = pair < pairs_needed;           // uniform per wave
-    const int n = lane & 31, g = lane >> 5;          // value product: head / feature n, half g
-    const int c = lane & 15, qd = lane >> 4;         // logits: head 16 hh + c, tokens 16 th + 4 qd + i
-    uint32_t err = 0;
+    const int st = w & (kSaStreams - 1), gi = w / kSaStreams;  // stream, head group of the set
+    const int n = lane & 15, kg = lane >> 4;
+    const int h0 = (hs * G + gi) * kSaHeads;
+    const bool live = h0 < p.heads;                    // uniform: a set's last group may hold no heads
 
-    // Cache rows of the split's indices, resolved once through the block table.
+    // Cache rows of the split's indices, resolved once through the block table (-1: none): all
+    // index loads, then the query's, then all table loads, so that the latencies overlap.
     const int span = kTopK / splits;
+    constexpr int kIt = kTopK / kThreads;
     const int* idx_row = p.indices + static_cast<size_t>(r) * kTopK + sp * span;
+    const int* table = p.block_table + static_cast<size_t>(b) * p.max_blocks;
     const int capacity = p.max_blocks * kBlockTokens;
-    for (int i = tid; i < span; i += kThreads) {
-        const int t = idx_row[i];
-        int row = -1;
-        if (t >= capacity) {
-            err |= KVIP_STATUS_BAD_TOKEN;
-        } else if (t >= 0) {
-            const int blk = p.block_table[static_cast<size_t>(b) * p.max_blocks + (t >> 7)];
-            if (static_cast<unsigned>(blk) < static_cast<unsigned>(p.num_blocks)) {
-                row = blk * kBlockTokens + (t & 127);
-            } else {
-                err |= KVIP_STATUS_BAD_BLOCK;
+    int idx[kIt];
+#pragma unroll
+    for (int i = 0; i < kIt; ++i) idx[i] = idx_row[min(i * kThreads + tid, span - 1)];
+    // Query of head h0 + n (heads past p.heads read another one's; their outputs are not written). The
+    // streams share the work: wave st takes scale group st, the 32 features that the lane's key bytes of
+    // that group are (pieces 8 st + kg and 8 st + 4 + kg), and rope piece 4 (st & 1) + kg.
+    v4i qraw[4], qrope;
+    {
+        const uint16_t* q = p.query + (static_cast<size_t>(r) * p.heads + min(h0 + n, p.heads - 1)) * kKeyDim;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            qraw[x] = *reinterpret_cast<const v4i*>(q + st * 128 + (x >> 1) * 64 + kg * 16 + (x & 1) * 8);
+        }
+        qrope = *reinterpret_cast<const v4i*>(q + kValueDim + (st & 1) * 32 + kg * 8);
+    }
+    uint32_t err = 0;
+    {
+        int blk[kIt];
+#pragma unroll
+        for (int i = 0; i < kIt; ++i) blk[i] = table[min(max(idx[i], 0), capacity - 1) >> 7];
+#pragma unroll
+        for (int i = 0; i < kIt; ++i) {
+            const bool ok = static_cast<unsigned>(blk[i]) < static_cast<unsigned>(p.num_blocks);
+            const bool in = idx[i] >= 0 && idx[i] < capacity;
+            err |= idx[i] >= capacity ? KVIP_STATUS_BAD_TOKEN : (in && !ok ? KVIP_STATUS_BAD_BLOCK : 0u);
+            if (i * kThreads + tid < span) {
+                s_row[i * kThreads + tid] = in && ok ? blk[i] * kBlockTokens + (idx[i] & 127) : -1;
             }
         }
-        s_row[i] = row;
     }
-
-    // Query fragments (B operand of the logits): head 32 pair + 16 hh + c, features
-    // 32 s + 8 qd .. + 8; heads past p.heads read as zero.
-    bf16x8 qf[kKSteps];
-    {
-        const int h = pair * 32 + 16 * hh + c;
-        const bool hl = live && h < p.heads;
-        const uint16_t* q = p.query + (static_cast<size_t>(r) * p.heads + (hl ? h : 0)) * kKeyDim + qd * 8;
+    f32x4 o[kBlocks];
 #pragma unroll
-        for (int s = 0; s < kKSteps; ++s) {
-            const v4i v = hl ? *reinterpret_cast<const v4i*>(q + s * 32) : v4i{0, 0, 0, 0};
-            qf[s] = as_bf16x8(v);
-        }
-    }
-    v16f o[kBlocks];
-#pragma unroll
-    for (int t = 0; t < kBlocks; ++t) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[t][i] = 0.f;
-    }
-    // Reference maxima (natural-log units) of head 16 hh + c ("own") and 16 (1 - hh) + c:
-    // every wave of the group follows all 32 heads, from the same tile maxima in the same order.
-    float m_own = -INFINITY, m_oth = -INFINITY;
-    float l_sum = 0.f;        // this lane's share of the own head's probability sum
-    bool o_zero = true;       // no tile has been accumulated yet (uniform)
+    for (int t = 0; t < kBlocks; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY;  // reference maximum of head n, log2 units
+    float l_sum = 0.f;        // this lane's share of its probability sum
+    const float scale2 = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(p.scale * kLog2e)));
     __syncthreads();
 
-    // Staging map: thread (token group tg, nope slice pc) holds the 16 nope features
-    // 16 pc .. of kTokPer consecutive tokens; the tile's 256 rope pieces go to threads 0-255.
-    const int tg = tid >> 5, pc = tid & 31;
-    const int f0 = pc * 16;
-    v4i nope[kTokPer];
-    float sc[kTokPer];
-    v4i rope = v4i{0, 0, 0, 0};
-    auto row_base = [&](int row) {
-        return p.kv_cache + static_cast<int64_t>(row >> 7) * p.kv_block_stride +
-               static_cast<int64_t>(row & 127) * p.row_stride;
-    };
-    auto load_tile = [&](int k) {
-#pragma unroll
-        for (int u = 0; u < kTokPer; ++u) {
-            const int row = s_row[k * kPrTile + tg * kTokPer + u];
-            nope[u] = v4i{0, 0, 0, 0};
-            sc[u] = 0.f;
-            if (row >= 0) {
-                const uint8_t* base = row_base(row);
-                nope[u] = *reinterpret_cast<const v4i*>(base + f0);
-                sc[u] = *reinterpret_cast<const float*>(base + 640 + (pc >> 3) * 4);
-            }
-        }
-        if (tid < kPrTile * 8) {
-            const int row = s_row[k * kPrTile + (tid >> 3)];
-            rope = row >= 0 ? *reinterpret_cast<const v4i*>(row_base(row) + 512 + (tid & 7) * 16) : v4i{0, 0, 0, 0};
-        }
-    };
-    // Dequantisation to bf16: keys [nope * scale, rope] token-major into tile buffer kb. The
-    // values are the same nope * scale features, read feature-wise by the transpose loads.
-    auto stage_tile = [&](uint16_t* kb) {
-#pragma unroll
-        for (int u = 0; u < kTokPer; ++u) {
-            uint32_t out[8];  // features f0 + 2k, 2k + 1
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(nope[u][k], false);
-                const f32x2 cc = __builtin_amdgcn_cvt_pk_f32_fp8(nope[u][k], true);
-                out[2 * k] = pack_bf16(a[0] * sc[u], a[1] * sc[u]);
-                out[2 * k + 1] = pack_bf16(cc[0] * sc[u], cc[1] * sc[u]);
-            }
-            uint16_t* d = kb + (tg * kTokPer + u) * kPrKPitch + f0;
-            reinterpret_cast<v4i*>(d)[0] = v4i{static_cast<int>(out[0]), static_cast<int>(out[1]),
-                                               static_cast<int>(out[2]), static_cast<int>(out[3])};
-            reinterpret_cast<v4i*>(d)[1] = v4i{static_cast<int>(out[4]), static_cast<int>(out[5]),
-                                               static_cast<int>(out[6]), static_cast<int>(out[7])};
-        }
-        if (tid < kPrTile * 8) {
-            *reinterpret_cast<v4i*>(kb + (tid >> 3) * kPrKPitch + 512 + (tid & 7) * 8) = rope;
-        }
-    };
-    // Transpose-load address of this lane within a tile: in each 16-lane block (j = lane % 16)
-    // lane j reads 4 features of one token, and lane j of the result holds one feature of 4
-    // consecutive tokens: block G = lane / 16 covers features 16 (G % 2) .. + 16 of tokens
-    // 8 (G / 2) .. + 4 (and + 4 .. + 8 by a second load), i.e. the B operand lane (feature n,
-    // tokens 8 g .. + 8) of the value MFMA.
-    const int tr_off = (8 * g + ((lane & 15) >> 2)) * kPrKPitch + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    uint8_t* ring = s_mem + st * 2 * kNopeSlot;
+    uint8_t* rope = s_mem + kLdsRope + st * kRopeSlot;
+    uint8_t* scales = s_mem + kLdsScale + st * 2 * kScaleSlot;
+    int64_t* s_base = reinterpret_cast<int64_t*>(s_mem + kLdsBase) + st * kSaTile;
+    const uint32_t ring_lds = lds_addr(ring), rope_lds = lds_addr(rope), scales_lds = lds_addr(scales);
 
-    const int tiles = span / kPrTile;
-    load_tile(0);
-    stage_tile(s_k[0]);
-    if (tiles > 1) load_tile(1);
-    __syncthreads();  // s_k[0] holds tile 0
-    for (int k = 0; k < tiles; ++k) {
-        const uint16_t* kt = s_k[k & 1];
-        const bool more = k + 1 < tiles;
-        // Tokens of the tile that have a row (bit t: token t).
-        const uint32_t vmask =
-            static_cast<uint32_t>(__ballot(lane < kPrTile && s_row[k * kPrTile + (lane & 31)] >= 0));
-        float sv[4];
-        if (live) {
-            // Logits of tokens 16 th .. + 16 (M) and heads 16 hh .. + 16 (N) over all 576
-            // features: lane (head 16 hh + c) gets tokens 16 th + 4 qd + i.
-            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-            const uint16_t* kr = kt + (16 * th + c) * kPrKPitch + 8 * qd;
+    // Tokens of tile k that have a row (bit t: token t), and their row addresses to s_base (0: none; the
+    // waves of a stream write the same values).
+    auto describe = [&](int k) -> uint32_t {
+        const int ln = fresh(lane);
+        const int row = s_row[k * kSaTile + (ln & 31)];
+        if (ln < kSaTile) {
+            s_base[ln] = row < 0 ? 0
+                                   : reinterpret_cast<int64_t>(p.kv_cache) +
+                                         static_cast<int64_t>(row >> 7) * p.kv_block_stride +
+                                         static_cast<int64_t>(row & 127) * p.row_stride;
+        }
+        return static_cast<uint32_t>(__ballot(row >= 0));
+    };
+    // This wave's share (1 / G) of the loads of the described tile's nope bytes and scales into
+    // slot `slot`. LDS row t holds piece s ^ swz(t) at place s; scales sit as [group][token]. Tokens
+    // without a row get zero bytes and zero scales (their probabilities are zero, and zero times a
+    // stray NaN would not be).
+    constexpr uint32_t kAll = 0xFFFFFFFFu;
+    auto load_nope = [&](int slot, uint32_t have) {
+        const int ln = fresh(lane);
+        constexpr int kLoads = kSaTile / 2 / G;  // of tokens 2 v and 2 v + 1 each
+        const int from = ((ln & 31) ^ sa_swz(ln >> 5) ^ (G == 2 ? sa_swz(16) * gi : 0)) * 16;
+        const int v0 = gi * kLoads, g0 = gi * (2 / G);
+        const int64_t base = s_base[ln & 31];  // scales: groups 2 v and 2 v + 1 per load
+        const uint8_t* sc_src = reinterpret_cast<const uint8_t*>(base) + 640 + 8 * g0 + 4 * (ln >> 5);
+        const uint32_t sc_dst = scales_lds + slot * kScaleSlot + g0 * 256, dst = ring_lds + slot * kNopeSlot + v0 * 1024;
+        if (have == kAll) {
+            int64_t row[kLoads];  // every address first: one LDS latency, not one per load
 #pragma unroll
-            for (int s = 0; s < kKSteps; ++s) {
-                const bf16x8 kv = as_bf16x8(*reinterpret_cast<const v4i*>(kr + s * 32));
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qf[s], acc, 0, 0, 0);
+            for (int x = 0; x < kLoads; ++x) row[x] = s_base[2 * (v0 + x) + (ln >> 5)];
+#pragma unroll
+            for (int x = 0; x < kLoads; ++x) {
+                dma16(reinterpret_cast<const uint8_t*>(row[x]) + (from ^ (sa_swz(2 * x) * 16)), dst + x * 1024);
             }
+#pragma unroll
+            for (int x = 0; x < 2 / G; ++x) dma4(sc_src + 8 * x, sc_dst + x * 256);
+        } else {
+#pragma unroll 1
+            for (int x = 0; x < kLoads; ++x) {
+                const int64_t row = s_base[2 * (v0 + x) + (ln >> 5)];
+                if (row != 0) {
+                    dma16(reinterpret_cast<const uint8_t*>(row) + (from ^ (sa_swz(2 * x) * 16)), dst + x * 1024);
+                } else {
+                    *(__attribute__((address_space(3))) v4i*)(dst + x * 1024 + ln * 16) = v4i{0, 0, 0, 0};
+                }
+            }
+#pragma unroll 1
+            for (int x = 0; x < 2 / G; ++x) {
+                if (base != 0) dma4(sc_src + 8 * x, sc_dst + x * 256);
+                else *(__attribute__((address_space(3))) float*)(sc_dst + x * 256 + ln * 4) = 0.f;
+            }
+        }
+    };
+    // And of its rope features: LDS row t (128 bytes) holds piece s ^ (t / 2 % 8) at place s. A token
+    // without a row keeps stale bytes: its logits are replaced.
+    auto load_rope = [&] {
+        const int ln = fresh(lane);
+        constexpr int kLoads = kSaTile / 8 / G;  // of tokens 8 v .. 8 v + 7 each
+        int64_t row[kLoads];
+#pragma unroll
+        for (int x = 0; x < kLoads; ++x) row[x] = s_base[8 * (gi * kLoads + x) + (ln >> 3)];
+#pragma unroll
+        for (int x = 0; x < kLoads; ++x) {
+            const int piece = (ln & 7) ^ (((4 * x) & 7) ^ (ln >> 4));
+            if (row[x] != 0) {
+                dma16(reinterpret_cast<const uint8_t*>(row[x]) + kValueDim + piece * 16,
+                      rope_lds + (gi * kLoads + x) * 1024);
+            }
+        }
+    };
+    // Every load and LDS access of this wave is done, and (waves sharing a stream) of all waves.
+    auto settle = [&](bool loads) {
+        if (loads) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");
+        else asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+        if constexpr (G > 1) {
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" : : : "memory");
+        }
+    };
+
+    const int tiles = span / kSaTile;  // a multiple of the streams
+    uint32_t mask = describe(st);
+    load_nope(0, mask);
+    load_rope();
+    report(p.status, err);
+
+    // The query as two fp8 e4m3 terms, q = (hi + lo) * 2^e with one e per head and 128 features (the
+    // block scale of the MFMA): hi takes the upper four of bf16's eight significant bits, lo the rest. That is exact
+    // for features within 2^9 of their group's largest and off by at most 2^-17 of the largest for
+    // smaller ones; a group with an infinity or NaN gets the NaN scale.
+    // Wave st converts group st; the terms go through LDS (the ring's second slots, free until the
+    // first tile has landed) to the waves of the other streams.
+    v4i* s_qf = reinterpret_cast<v4i*>(s_mem + kNopeSlot) + gi * 256;  // + stream * 2 slots: its group's terms
+    int* s_qe = reinterpret_cast<int*>(s_mem + kLdsQuery);             // [group of heads][head][scale group]
+    {
+        uint32_t top = 0;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) {
+            const uint32_t v = static_cast<uint32_t>(qraw[x >> 2][x & 3]);
+            top = max(top, max(v & 0x7FFFu, (v >> 16) & 0x7FFFu));
+        }
+        top = static_cast<uint32_t>(rows4_max(static_cast<float>(top >> 7)));  // over the group's four lanes
+        const int e = max(static_cast<int>(top), 8);        // biased exponent of the largest
+        const float mul = __int_as_float((261 - e) << 23);  // 2^(134 - e): the largest below 2^8
+        v4i* dst = s_qf + st * (2 * kNopeSlot / 16) + lane;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {  // features of the lane's first, second piece
+            v4i hi, lo;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+                int h = 0, l = 0;
+#pragma unroll
+                for (int y = 0; y < 2; ++y) {
+                    const uint32_t v = static_cast<uint32_t>(qraw[2 * half + (x >> 1)][(x & 1) * 2 + y]);
+                    const float a = __uint_as_float(v << 16) * mul, c = __uint_as_float(v & 0xFFFF0000u) * mul;
+                    h = y ? __builtin_amdgcn_cvt_pk_fp8_f32(a, c, h, true) : __builtin_amdgcn_cvt_pk_fp8_f32(a, c, h, false);
+                    const f32x2 back = y ? __builtin_amdgcn_cvt_pk_f32_fp8(h, true) : __builtin_amdgcn_cvt_pk_f32_fp8(h, false);
+                    l = y ? __builtin_amdgcn_cvt_pk_fp8_f32(a - back[0], c - back[1], l, true)
+                          : __builtin_amdgcn_cvt_pk_fp8_f32(a - back[0], c - back[1], l, false);
+                }
+                hi[x] = h;
+                lo[x] = l;
+            }
+            dst[half * 64] = hi;
+            dst[(2 + half) * 64] = lo;
+        }
+        if (kg == 0) s_qe[(gi * kSaHeads + n) * kScaleGroups + st] = e == 255 ? 255 : e - 7;
+    }
+    v4i* s_rope = reinterpret_cast<v4i*>(s_mem + kLdsQuery + 2 * kSaHeads * kScaleGroups * 4) + gi * 64;
+    if (st == 0) s_qf[512 + lane] = qrope;  // past the terms of both head groups
+    if (st == 1) s_rope[lane] = qrope;
+    lds_sync();
+    v8i qh[kScaleGroups], ql[kScaleGroups];
+    int qscale = 0;  // byte g: E8M0 scale of group g
+#pragma unroll
+    for (int g = 0; g < kScaleGroups; ++g) {
+        const v4i* src = s_qf + g * (2 * kNopeSlot / 16) + lane;
+        const v4i a = src[0], c = src[64], d = src[128], f = src[192];
+        qh[g] = v8i{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+        ql[g] = v8i{d[0], d[1], d[2], d[3], f[0], f[1], f[2], f[3]};
+        qscale |= s_qe[(gi * kSaHeads + n) * kScaleGroups + g] << (8 * g);
+    }
+    const bf16x8 q_rope = __builtin_bit_cast(bf16x8, s_qf[512 + lane]);
+    lds_sync();  // the ring's second slots are free
+    int slot = 0;
+    for (int k = st; k < tiles; k += kSaStreams, slot ^= 1) {
+        const bool more = k + kSaStreams < tiles;
+        settle(true);  // the tile has landed; the other slot is free
+        uint32_t next = 0;
+        if (more) {
+            next = describe(k + kSaStreams);
+            load_nope(slot ^ 1, next);
+        }
+        // LDS addresses of this lane's reads, derived anew for each tile (held over the loop they
+        // would cost registers that the accumulators need). Keys: piece 4 j + kg of token 16 u + n; the
+        // XOR with 64 j moves between pieces. Values: block kg of a transpose load covers 16 features
+        // (one piece) of the 8 tokens that lane group kg holds probabilities of: 4 kg + 0 .. 3 and
+        // 16 + 4 kg + 0 .. 3.
+        const int ln = fresh(lane), tn = ln & 15, tk = ln >> 4;
+        const uint32_t ro = rope_lds + tn * 128 + ((tk ^ ((tn >> 1) & 7)) << 4);
+        const uint32_t ko = ring_lds + slot * kNopeSlot + tn * kValueDim + ((tk ^ sa_swz(tn)) << 4);
+        const int vt = 4 * tk + ((tn >> 1) & 3) + 16 * (tn >> 3);
+        const uint32_t vo = ring_lds + slot * kNopeSlot + vt * kValueDim + (sa_swz(vt) << 4) + 8 * (ln & 1);
+        const uint32_t sl = scales_lds + slot * kScaleSlot + 16 * tk;  // scales of tokens 4 kg .. + 3
+
+        // Logits [tokens, heads], lane: tokens 16 u + 4 kg + i of head n. Rope first, whose buffer
+        // then takes the next tile's rope.
+        f32x4 sv[2];
+        {
+            const v4i q1 = *(LdsV4i)lds_addr(s_rope + ln);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const v4i k0 = *(LdsV4i)(ro + u * 16 * 128), k1 = *(LdsV4i)((ro ^ 64) + u * 16 * 128);
+                sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k0), q_rope,
+                                                                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k1),
+                                                                __builtin_bit_cast(bf16x8, q1), sv[u], 0, 0, 0);
+            }
+        }
+        settle(false);
+        if (more) load_rope();
+        if (live) {
+            // One scale group of 16 tokens per step (i: token half i / 4, group i % 4), its key bytes read
+            // one step ahead; the raw fp8 bytes are the A operand.
+            auto key = [&](int i) {
+                const uint32_t at = ko ^ ((i & 3) * 128) ^ (sa_swz(16 * (i >> 2)) * 16);
+                const v4i x = *(LdsV4i)(at + (i >> 2) * 16 * kValueDim);
+                const v4i y = *(LdsV4i)((at ^ 64) + (i >> 2) * 16 * kValueDim);
+                return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+            };
+            v8i kv[2] = {key(0), v8i{}};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int u = i >> 2, g = i & 3;
+                const f32x4 s4 = *(LdsF32x4)(sl + (g * kSaTile + 16 * u) * 4);
+                if (i + 1 < 8) kv[(i + 1) & 1] = key(i + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                f32x4 part = sa_mma8(kv[i & 1], qh[g], f32x4{0.f, 0.f, 0.f, 0.f}, g, qscale);
+                part = sa_mma8(kv[i & 1], ql[g], part, g, qscale);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sv[u][e] = fmaf(part[e], s4[e], sv[u][e]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // Softmax: pr = 2^(logit - m), the logits of tokens without a row at -inf.
+            float pr[8];
             float mx = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float v = acc[i] * p.scale;
-                if (!((vmask >> (16 * th + 4 * qd + i)) & 1u)) v = -INFINITY;
-                sv[i] = v;
-                mx = fmaxf(mx, v);
-            }
-            mx = rows4_max(mx);  // the head's maximum over this wave's 16 tokens
-            if (qd == 0) s_m[gi][th][16 * hh + c] = mx;
-        }
-        __syncthreads();  // both token halves' maxima of every head in s_m
-        if (live) {
-            const float t_own = fmaxf(s_m[gi][0][16 * hh + c], s_m[gi][1][16 * hh + c]);
-            const float t_oth = fmaxf(s_m[gi][0][16 * (1 - hh) + c], s_m[gi][1][16 * (1 - hh) + c]);
-            const bool n_own = t_own > m_own + kPrMargin;  // also the first finite maximum
-            const bool n_oth = t_oth > m_oth + kPrMargin;
-            if (__ballot(n_own || n_oth) != 0ull) {  // the same decision in every wave of the group
-                const float new_own = n_own ? t_own : m_own, new_oth = n_oth ? t_oth : m_oth;
-                const float a_own = (m_own == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_own - new_own) * kPrLog2e);
-                const float a_oth = (m_oth == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f((m_oth - new_oth) * kPrLog2e);
-                l_sum *= n_own ? a_own : 1.f;
-                if (!o_zero) {
-                    if (qd == 0) {
-                        s_h[w][16 * hh + c] = n_own ? a_own : 1.f;
-                        s_h[w][16 * (1 - hh) + c] = n_oth ? a_oth : 1.f;
-                    }
-                    // Wave-local: this wave's LDS writes precede its reads.
-                    f32x4 a4[4];
+            for (int i = 0; i < 8; ++i) pr[i] = sv[i >> 2][i & 3] * scale2;
+            if (mask != kAll) {
+                const uint32_t mine = mask >> (4 * tk);
 #pragma unroll
-                    for (int qq = 0; qq < 4; ++qq) a4[qq] = *reinterpret_cast<const f32x4*>(&s_h[w][8 * qq + 4 * g]);
-#pragma unroll
-                    for (int t = 0; t < kBlocks; ++t) {
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) o[t][i] *= a4[i >> 2][i & 3];
-                    }
-                }
-                m_own = new_own;
-                m_oth = new_oth;
-            }
-            const float bias = m_own == -INFINITY ? 0.f : -m_own * kPrLog2e;
-            const float p0 = __builtin_amdgcn_exp2f(fmaf(sv[0], kPrLog2e, bias));
-            const float p1 = __builtin_amdgcn_exp2f(fmaf(sv[1], kPrLog2e, bias));
-            const float p2 = __builtin_amdgcn_exp2f(fmaf(sv[2], kPrLog2e, bias));
-            const float p3 = __builtin_amdgcn_exp2f(fmaf(sv[3], kPrLog2e, bias));
-            l_sum += (p0 + p1) + (p2 + p3);
-            *reinterpret_cast<i32x2*>(s_p[gi] + (16 * hh + c) * kPrPPitch + 16 * th + 4 * qd) =
-                i32x2{static_cast<int>(pack_bf16(p0, p1)), static_cast<int>(pack_bf16(p2, p3))};
-        }
-        __syncthreads();  // the group's probabilities in s_p
-        if (live) {
-            // Value product: features kVPart hf + 32 t + n; K step s2 covers tokens 16 s2 + 8 g
-            // .. + 8 of head n (A: probabilities, B: transpose loads of the key tile).
-            bf16x8 pa[2];
-#pragma unroll
-            for (int s2 = 0; s2 < 2; ++s2) {
-                pa[s2] = as_bf16x8(*reinterpret_cast<const v4i*>(s_p[gi] + n * kPrPPitch + 16 * s2 + 8 * g));
-            }
-#pragma unroll
-            for (int t = 0; t < kBlocks; ++t) {
-                const uint16_t* vr = kt + tr_off + hf * kVPart + t * 32;
-#pragma unroll
-                for (int s2 = 0; s2 < 2; ++s2) {
-                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s*)(vr + 16 * s2 * kPrKPitch));
-                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                        (__attribute__((address_space(3))) v4s*)(vr + (16 * s2 + 4) * kPrKPitch));
-                    const bf16x8 vb = __builtin_bit_cast(bf16x8, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
-                    o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[s2], vb, o[t], 0, 0, 0);
+                for (int i = 0; i < 8; ++i) {
+                    if (!((mine >> (16 * (i >> 2) + (i & 3))) & 1u)) pr[i] = -INFINITY;
                 }
             }
-            o_zero = false;
-            // The next tile's staging beside this tile's value MFMAs (inside the branch, so
-            // the scheduler can interleave them), then the loads of the tile after it.
-            if (more) {
-                stage_tile(s_k[(k + 1) & 1]);
-                if (k + 2 < tiles) load_tile(k + 2);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) mx = fmaxf(mx, pr[i]);
+            mx = rows4_max(mx);
+            const bool raise = mx > m_run + kSaMargin;  // also the first finite maximum
+            if (__ballot(raise) != 0ull) {
+                const float m_new = raise ? mx : m_run;
+                const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+                const float a = raise ? alpha : 1.f;
+                l_sum *= a;
+#pragma unroll
+                for (int t = 0; t < kBlocks; ++t) o[t] *= a;
+                m_run = m_new;
             }
-        } else if (more) {
-            stage_tile(s_k[(k + 1) & 1]);
-            if (k + 2 < tiles) load_tile(k + 2);
+            const float bias = m_run == -INFINITY ? 0.f : -m_run;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                pr[i] = __builtin_amdgcn_exp2f(pr[i] + bias);
+                l_sum += pr[i];
+            }
+            // Value product [features, heads]: the transpose loads of kAhead blocks ahead of the MFMAs
+            // of the kAhead before them; each scale group's probabilities as its first block comes up.
+            constexpr int kAhead = G == 1 ? 4 : 2;  // two waves per SIMD have no registers for more
+            auto value = [&](int t) {
+                return __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsI32x2)((vo ^ ((t & 15) * 16)) + (t & 16) * 16));
+            };
+            i32x2 raw[2][kAhead];
+#pragma unroll
+            for (int i = 0; i < kAhead; ++i) raw[0][i] = value(i);
+            bf16x8 pb;
+#pragma unroll
+            for (int t = 0; t < kBlocks; t += kAhead) {
+                const int now = t / kAhead & 1;
+                if (t + kAhead < kBlocks) {
+#pragma unroll
+                    for (int i = 0; i < kAhead; ++i) raw[now ^ 1][i] = value(t + kAhead + i);
+                }
+                if (t % 8 == 0) {
+                    v4i packed;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const f32x4 s4 = *(LdsF32x4)(sl + (t / 8 * kSaTile + 16 * u) * 4);
+                        packed[2 * u] = static_cast<int>(pack_bf16(pr[4 * u] * s4[0], pr[4 * u + 1] * s4[1]));
+                        packed[2 * u + 1] = static_cast<int>(pack_bf16(pr[4 * u + 2] * s4[2], pr[4 * u + 3] * s4[3]));
+                    }
+                    pb = __builtin_bit_cast(bf16x8, packed);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < kAhead; ++i) {
+                    const i32x2 x = raw[now][i];
+                    o[t + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16(x[0], x[1]), pb, o[t + i], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
-        __syncthreads();  // tile k + 1 staged; tile k's buffer, s_m and s_p free
+        mask = next;
     }
 
-    // Probability sums: over the lane's four token rows, then the two token halves; then the
-    // split's partial record (max, sum, unnormalised output per head) or the normalised
-    // output. Output lane (feature kVPart hf + 32 t + n) holds heads 32 pair + 8 (i / 4) +
-    // 4 g + i % 4 of o[t][i].
-    if (live) {
-        const float l = rows4_sum(l_sum);
-        if (qd == 0) s_m[gi][th][16 * hh + c] = l;
+    // Merge of the streams: with the maximum M over them, out = sum_w 2^(m_w - M) o_w / l and
+    // l = sum_w 2^(m_w - M) l_w, 512 / G features at a time through LDS.
+    const float l_all = rows4_sum(l_sum);
+    float* s_m = reinterpret_cast<float*>(s_mem + kLdsScale);  // [wave][head], then the sums
+    float* s_f = s_m + 2 * kWaves * kSaHeads;                  // [wave][head]: factor of the wave's output
+    float* buf = reinterpret_cast<float*>(s_mem);              // [wave][head][features]
+    constexpr int kPitch = kValueDim / G + 4;
+    static_assert(kWaves * kSaHeads * kPitch * 4 <= kLdsScale, "merge buffer inside ring and rope");
+    __syncthreads();  // every wave is done with its ring, rope and scales
+    if (kg == 0) {
+        s_m[w * kSaHeads + n] = m_run;
+        s_m[(kWaves + w) * kSaHeads + n] = l_all;
     }
-    __syncthreads();
-    if (live) {
-        const float l_n = s_m[gi][0][n] + s_m[gi][1][n];  // head n of the group
-        const int groups = (p.heads + kSaHeads - 1) / kSaHeads;
-        if (splits > 1) {
-            if (hf == 0 && g == 0) {
-                // Wave 0 (hh = 0) holds head c as its own and 16 + c as the other.
-                const int h = pair * 32 + n;
-                if (h < p.heads) {
-                    float* ws = p.workspace + ((static_cast<size_t>(r) * groups + h / kSaHeads) * splits + sp) * kPartial;
-                    ws[h % kSaHeads] = n < 16 ? m_own : m_oth;
-                    ws[kSaHeads + h % kSaHeads] = l_n;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        if (g > 0) __syncthreads();  // the features before have been read
+#pragma unroll
+        for (int t = 0; t < kBlocks / G; ++t) {
+            *reinterpret_cast<f32x4*>(buf + (w * kSaHeads + n) * kPitch + t * 16 + 4 * kg) = o[g * (kBlocks / G) + t];
+        }
+        __syncthreads();
+        if (g == 0) {
+            if (tid < kSaHeads * G) {
+                const int w0 = tid / kSaHeads * kSaStreams, hn = tid % kSaHeads;  // the head's waves
+                float m = -INFINITY;
+#pragma unroll
+                for (int v = 0; v < kSaStreams; ++v) m = fmaxf(m, s_m[(w0 + v) * kSaHeads + hn]);
+                float l = 0.f, f[kSaStreams];
+#pragma unroll
+                for (int v = 0; v < kSaStreams; ++v) {
+                    f[v] = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(s_m[(w0 + v) * kSaHeads + hn] - m);
+                    l += f[v] * s_m[(kWaves + w0 + v) * kSaHeads + hn];
                 }
+                const int h = hs * G * kSaHeads + tid;
+                float inv = 1.f;
+                if (splits == 1) {
+                    inv = l > 0.f ? 1.f / l : 0.f;
+                } else if (h < p.heads) {
+                    float* ml = p.workspace + static_cast<size_t>(p.rows) * p.heads * splits * kValueDim +
+                                ((static_cast<size_t>(r) * p.heads + h) * splits + sp) * 2;
+                    ml[0] = m;
+                    ml[1] = l;
+                }
+#pragma unroll
+                for (int v = 0; v < kSaStreams; ++v) s_f[(w0 + v) * kSaHeads + hn] = f[v] * inv;
             }
+            __syncthreads();
+        }
+        // Thread: features f .. + 4 of every kStep-th head; consecutive threads on consecutive features.
+        constexpr int kPerHead = kValueDim / G / 4;
+        constexpr int kStep = kThreads / kPerHead;
+        const int f = tid % kPerHead * 4;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int h = pair * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-                if (h >= p.heads) continue;
-                float* ws = p.workspace + ((static_cast<size_t>(r) * groups + h / kSaHeads) * splits + sp) * kPartial +
-                            2 * kSaHeads + (h % kSaHeads) * kValueDim + hf * kVPart + n;
+        for (int hl = tid / kPerHead; hl < kSaHeads * G; hl += kStep) {
+            const int w0 = hl / kSaHeads * kSaStreams;
+            f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int t = 0; t < kBlocks; ++t) ws[t * 32] = o[t][i];
+            for (int x = 0; x < kSaStreams; ++x) {
+                const int at = (w0 + x) * kSaHeads + hl % kSaHeads;
+                v += s_f[at] * *reinterpret_cast<const f32x4*>(buf + at * kPitch + f);
             }
-        } else {
-            if (g == 0) s_h[w][n] = l_n > 0.f ? 1.f / l_n : 0.f;
-            f32x4 inv[4];
-#pragma unroll
-            for (int qq = 0; qq < 4; ++qq) inv[qq] = *reinterpret_cast<const f32x4*>(&s_h[w][8 * qq + 4 * g]);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int h = pair * 32 + 8 * (i >> 2) + 4 * g + (i & 3);
-                if (h >= p.heads) continue;
-                float* out = p.output + (static_cast<size_t>(r) * p.heads + h) * kValueDim + hf * kVPart + n;
-#pragma unroll
-                for (int t = 0; t < kBlocks; ++t) out[t * 32] = o[t][i] * inv[i >> 2][i & 3];
+            const int h = hs * G * kSaHeads + hl;
+            if (h < p.heads) {
+                const size_t rh = static_cast<size_t>(r) * p.heads + h;
+                float* out = splits == 1 ? p.output + rh * kValueDim : p.workspace + (rh * splits + sp) * kValueDim;
+                *reinterpret_cast<f32x4*>(out + g * (kValueDim / G) + f) = v;
             }
         }
     }
-    report(p.status, err);
 }
 
-// Merge of the splits: workgroup (row, head group, 64-feature chunk).
-__global__ __launch_bounds__(kSaThreads) void sparse_attention_merge_kernel(const KvipSparseAttnArgs p) {
-    __shared__ float s_w[kMaxSplits][kSaHeads];
-    __shared__ float s_inv[kSaHeads];
-    const int groups = (p.heads + kSaHeads - 1) / kSaHeads;
-    const int splits = sa_splits(p.rows, sa_sets(p.heads));
-    const int unit = blockIdx.x / 8, part = blockIdx.x % 8;
-    const int r = unit / groups, h0 = (unit % groups) * kSaHeads;
-    const float* ws = p.workspace + static_cast<size_t>(unit) * splits * kPartial;
-    const int tid = threadIdx.x;
-    if (tid < kSaHeads) {
-        float m = -INFINITY;
-        for (int s = 0; s < splits; ++s) m = fmaxf(m, ws[s * kPartial + tid]);
-        float l = 0.f;
-        for (int s = 0; s < splits; ++s) {
-            const float wgt = m == -INFINITY ? 0.f : __expf(ws[s * kPartial + tid] - m);
-            s_w[s][tid] = wgt;
-            l += wgt * ws[s * kPartial + kSaHeads + tid];
-        }
-        s_inv[tid] = l > 0.f ? 1.f / l : 0.f;
+// Merge of the splits: 128 threads per (row, head), four features each; every load is issued before the
+// first is used (one memory latency, whatever the split count).
+template <int SPLITS>
+__global__ __launch_bounds__(256) void sparse_attention_merge_kernel(const KvipSparseAttnArgs p) {
+    const int64_t rh = static_cast<int64_t>(blockIdx.x) * 2 + (threadIdx.x >> 7);
+    if (rh >= static_cast<int64_t>(p.rows) * p.heads) return;
+    const int f = (threadIdx.x & 127) * 4;
+    const float* ws = p.workspace + rh * SPLITS * kValueDim + f;
+    const float* ml = p.workspace + static_cast<size_t>(p.rows) * p.heads * SPLITS * kValueDim + rh * SPLITS * 2;
+    f32x4 part[SPLITS];
+    f32x2 sums[SPLITS];
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s) sums[s] = *reinterpret_cast<const f32x2*>(ml + 2 * s);
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s) part[s] = *reinterpret_cast<const f32x4*>(ws + s * kValueDim);
+    float m = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s) m = fmaxf(m, sums[s][0]);
+    float l = 0.f;
+    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s) {
+        const float wgt = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sums[s][0] - m);
+        l += wgt * sums[s][1];
+        v += wgt * part[s];
     }
-    __syncthreads();
-    // One thread per 4 features of one head (16 heads x 64 features = 256 float4).
-    const int h = tid / 16, col = part * 64 + (tid % 16) * 4;
-    if (h0 + h < p.heads) {
-        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int s = 0; s < splits; ++s) {
-            const f32x4 o = *reinterpret_cast<const f32x4*>(ws + s * kPartial + 2 * kSaHeads + h * kValueDim + col);
-            v += s_w[s][h] * o;
-        }
-        *reinterpret_cast<f32x4*>(p.output + (static_cast<size_t>(r) * p.heads + h0 + h) * kValueDim + col) =
-            v * s_inv[h];
-    }
+    *reinterpret_cast<f32x4*>(p.output + rh * kValueDim + f) = v * (l > 0.f ? 1.f / l : 0.f);
+}
+
+template <int SPLITS>
+void launch_merge(const KvipSparseAttnArgs& a, hipStream_t stream) {
+    const int64_t pairs = (static_cast<int64_t>(a.rows) * a.heads + 1) / 2;
+    hipLaunchKernelGGL(sparse_attention_merge_kernel<SPLITS>, dim3(static_cast<unsigned>(pairs)), dim3(256), 0, stream, a);
 }
 
 }  // namespace
 
 uint64_t sparse_attention_workspace_bytes(int rows, int heads) {
     if (rows < 1 || heads < 1) return 0;
-    const int groups = (heads + kSaHeads - 1) / kSaHeads;
-    const int splits = sa_splits(rows, sa_sets(heads));
-    return splits > 1 ? static_cast<uint64_t>(rows) * groups * splits * kPartial * sizeof(float) : 0;
+    const int splits = sa_splits(rows, heads);
+    return splits > 1 ? static_cast<uint64_t>(rows) * heads * splits * kPartial * sizeof(float) : 0;
 }
 
 uint32_t validate_sparse_attention(const KvipSparseAttnArgs* a) {
@@ -782,22 +665,21 @@ uint32_t validate_sparse_attention(const KvipSparseAttnArgs* a) {
 extern "C" uint32_t kvip_hip_sparse_attention(const KvipSparseAttnArgs* args, void* stream) {
     const uint32_t rc = kvip::validate_sparse_attention(args);
     if (rc != KVIP_OK) return rc;
-    const int groups = (args->heads + kvip::kSaHeads - 1) / kvip::kSaHeads;
     const int sets = kvip::sa_sets(args->heads);
-    const int splits = kvip::sa_splits(args->rows, sets);
+    const int splits = kvip::sa_splits(args->rows, args->heads);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid(((args->rows + 7) / 8) * 8 * sets * splits);
-    if (kvip::sa_pairs(args->heads)) {
-        hipLaunchKernelGGL((kvip::sparse_attention_pair_kernel<kvip::kPrGroups, kvip::kPrSplit>), grid,
-                           dim3(kvip::kPrGroups * kvip::kPrSplit * 64), 0, s, *args);
-    } else if (kvip::sa_group_set(args->heads) == 2) {
-        hipLaunchKernelGGL(kvip::sparse_attention_kernel<2>, grid, dim3(2 * kvip::kSaThreads), 0, s, *args);
+    const dim3 grid((args->rows * splits + 7) / 8 * 8 * sets);
+    if (args->heads > 16) {
+        hipLaunchKernelGGL(kvip::sparse_attention_kernel<2>, grid, dim3(512), 0, s, *args, splits);
     } else {
-        hipLaunchKernelGGL(kvip::sparse_attention_kernel<1>, grid, dim3(kvip::kSaThreads), 0, s, *args);
+        hipLaunchKernelGGL(kvip::sparse_attention_kernel<1>, grid, dim3(256), 0, s, *args, splits);
     }
-    if (splits > 1) {
-        hipLaunchKernelGGL(kvip::sparse_attention_merge_kernel, dim3(args->rows * groups * 8), dim3(kvip::kSaThreads),
-                           0, s, *args);
+    switch (splits) {
+        case 2: kvip::launch_merge<2>(*args, s); break;
+        case 4: kvip::launch_merge<4>(*args, s); break;
+        case 8: kvip::launch_merge<8>(*args, s); break;
+        case 16: kvip::launch_merge<16>(*args, s); break;
+        default: break;
     }
     return static_cast<uint32_t>(hipGetLastError());
 }

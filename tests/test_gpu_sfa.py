@@ -219,3 +219,49 @@ def test_sparse_attention_graph_replay(torch_gpu, heads):
         _ = (q.float() * 2).sum().item()  # eager work between replays
     op.output.zero_()
     assert torch.equal(op(), eager)
+
+
+@pytest.mark.parametrize("heads,rows,per_request", [(1, 1, 1), (16, 3, 1), (17, 40, 2), (33, 6, 1), (48, 200, 4)])
+def test_sparse_attention_edges_against_64_bits(torch_gpu, heads, rows, per_request):
+    """Partly filled head groups and sets, every split count (16 splits for one row down to
+    none for 200), rows with a single index, with whole tiles of absent indices and with
+    all 2048, queries whose features span 2^-20 .. 2^3 within a scale group, and a cache whose
+    block 0, row 0 (never selected) is NaN throughout. Each probability is rounded once to
+    bf16 (2^-9 relative), everything else is fp32: the error is held to twice that bound,
+    2^-8 sum_j p_j |v_j| / sum_j p_j per feature."""
+    torch = torch_gpu
+    gen = torch.Generator(device="cuda").manual_seed(heads * 1000 + rows)
+    batch, max_blocks = rows // per_request, 20
+    blocks = 64
+    values = torch.randn((blocks * 128, 4, 128), generator=gen, device="cuda")
+    scales = torch.rand((blocks * 128, 4), generator=gen, device="cuda") * 0.02 + 0.0005
+    kv = torch.empty((blocks * 128, ROW), dtype=torch.uint8, device="cuda")
+    codes = (values * 60).to(torch.float8_e4m3fn)
+    kv[:, :512] = codes.view(torch.uint8).view(-1, 512)
+    rope = torch.randn((blocks * 128, 64), generator=gen, device="cuda").to(torch.bfloat16)
+    kv[:, 512:640] = rope.view(torch.uint8)
+    kv[:, 640:] = scales.view(torch.uint8)
+    kv[0] = 0x7F  # NaN codes; rope and scales 0x7F7F..: huge
+    kv[0, 640:] = torch.full((4,), float("nan"), device="cuda").view(torch.uint8)
+    table = torch.stack([torch.randperm(blocks - 1, generator=gen, device="cuda")[:max_blocks] + 1 for _ in range(batch)])
+    table = table.to(torch.int32)
+    idx = torch.randint(0, max_blocks * 128, (rows, TOPK), generator=gen, device="cuda", dtype=torch.int32)
+    idx[0, 1:] = -1
+    if rows > 1:
+        idx[1, 64:1024] = -1
+        idx[1, 1500::3] = -1
+    span = torch.randint(-20, 4, (rows, heads, 576), generator=gen, device="cuda").float()
+    q = (torch.randn((rows, heads, 576), generator=gen, device="cuda") * torch.exp2(span)).to(torch.bfloat16)
+    say(f"case edges heads={heads} rows={rows}")
+    out = sparse_attention(q, kv.view(blocks, 128, ROW), table, idx, SCALE, rows_per_request=per_request).double()
+    key = torch.cat([(codes.double() * scales.double()[:, :, None]).view(-1, 512), rope.double()], dim=1)
+    worst = 0.0
+    for r in sorted({0, 1 % rows, rows // 2, rows - 1}):
+        t = idx[r][idx[r] >= 0].long()
+        k = key[table[r // per_request].long()[t // 128] * 128 + t % 128].contiguous()
+        prob = torch.softmax(q[r].double() @ k.T.contiguous() * SCALE, dim=1)
+        want = prob @ k[:, :512].contiguous()
+        bound = 2.0 ** -8 * (prob @ k[:, :512].abs().contiguous()) + 1e-7
+        worst = max(worst, ((out[r] - want).abs() / bound).max().item())
+    say(f"  worst error over its bound: {worst:.3f}")
+    assert worst <= 1.0
