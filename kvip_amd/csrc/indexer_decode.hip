@@ -44,6 +44,7 @@ constexpr int kTileTokens = 32;
 constexpr int kTilesPerWave = 4;                                        // chunked kernel
 constexpr int kChunkTokens = kLiWaves * kTilesPerWave * kTileTokens;    // 512
 constexpr int kStreamMaxBatch = 2048;
+constexpr int kCombineWaves = 128;
 // Tiles per streaming sub-segment: its keys fit the wave's 4 KiB LDS key strip (and
 // its page ids one register per lane).
 template <int RPR>
@@ -178,6 +179,7 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
     __shared__ uint32_t s_scan[kLiWaves];
     __shared__ __align__(16) float s_w[kLiWaves][RPR * HEADS];
     __shared__ uint32_t s_hist[kLiWaves][RPR * 256];
+    __shared__ int s_req[kLiWaves];  // request of the histogram each wave still holds, -1: none
     __shared__ __align__(16) uint8_t s_tile[kLiWaves][T::BYTES];
     constexpr int SEG = kSegmentTiles<RPR>;
     __shared__ __align__(16) uint16_t s_keys[kLiWaves][RPR * SEG * kTileTokens];
@@ -212,9 +214,16 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
     const int total_tiles = s_prefix[p.batch];
     const int64_t nw = static_cast<int64_t>(gridDim.x) * kLiWaves;
     const int64_t w = static_cast<int64_t>(blockIdx.x) * kLiWaves + __builtin_amdgcn_readfirstlane(wave);
-    int t = static_cast<int>(total_tiles * w / nw);
-    const int t_end = static_cast<int>(total_tiles * (w + 1) / nw);
-    if (t >= t_end) return;  // no barriers follow: waves run independently from here
+    int t, t_end;
+    if (total_tiles <= nw) {  // a tile per wave, packed into the first workgroups (fewer histogram adds)
+        t = static_cast<int>(w);
+        t_end = min(t + 1, total_tiles);
+        if (blockIdx.x * kLiWaves >= static_cast<unsigned>(total_tiles)) return;  // uniform for the workgroup
+    } else {
+        t = static_cast<int>(total_tiles * w / nw);
+        t_end = static_cast<int>(total_tiles * (w + 1) / nw);
+    }
+    // The waves run independently from here (to the barrier before combined histogram adds).
     int lo = 0, hi = p.batch - 1;  // largest b with s_prefix[b] <= t
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -230,6 +239,10 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
     float* w_rows = s_w[wave];
     uint32_t* hist = s_hist[wave];
     uint32_t err = 0;
+    int held = -1;
+    // Many waves per request: the workgroup's waves add the histograms they end with as one (adds to a
+    // row serialise at ~10 ns each; one row of 32768 tokens 19.5 -> 11.1 us, of 131072 32.3 -> 16.2).
+    const bool combine = nw > kCombineWaves * p.batch;
 
     while (t < t_end) {  // one segment = this wave's tiles of request b
         while (s_prefix[b + 1] <= t) ++b;
@@ -292,7 +305,8 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
             __builtin_amdgcn_sched_barrier(0);
             issue(1, b1, k1);
             __builtin_amdgcn_sched_barrier(0);
-            for (int i = 0; i < cnt; i += 3) {
+            int i = 0;
+            for (; i + 3 <= cnt; i += 3) {
                 issue(i + 2, b2, k2);
                 __builtin_amdgcn_sched_barrier(0);
                 compute(i, b0, k0);
@@ -303,6 +317,8 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
                 __builtin_amdgcn_sched_barrier(0);
                 compute(i + 2, b2, k2);
             }
+            if (i < cnt) compute(i, b0, k0);
+            if (i + 1 < cnt) compute(i + 1, b1, k1);
             // Flush the sub-segment's keys: 8 bytes per lane per store, coalesced. Keys past
             // `valid` stay inside the row and are never read.
 #pragma unroll
@@ -315,12 +331,37 @@ __global__ __launch_bounds__(kLiThreads) void indexer_stream_kernel(const KvipIn
             }
             t += cnt;
         }
-        // Flush the request's histogram.
-        for (int i = lane; i < RPR * 256; i += 64) {
-            const uint32_t c = hist[i];
-            if (c != 0u) {
-                atomicAdd(&p.histogram[static_cast<size_t>(b) * RPR * 256 + i], c);
-                hist[i] = 0u;
+        // Flush the request's histogram (the last one may be held for the workgroup's sum).
+        if (combine && t >= t_end) {
+            held = b;
+        } else {
+            for (int i = lane; i < RPR * 256; i += 64) {
+                const uint32_t c = hist[i];
+                if (c != 0u) {
+                    atomicAdd(&p.histogram[static_cast<size_t>(b) * RPR * 256 + i], c);
+                    hist[i] = 0u;
+                }
+            }
+        }
+    }
+    if (!combine) {
+        report(p.status, err);
+        return;
+    }
+    // The held histograms, summed over consecutive waves of one request (the ranges are in
+    // order, so the requests are too).
+    if (lane == 0) s_req[wave] = held;
+    __syncthreads();
+    for (int i = tid; i < RPR * 256; i += kLiThreads) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (int v = 0; v < kLiWaves; ++v) {
+            const int req = s_req[v];
+            if (req < 0) continue;  // uniform
+            sum += s_hist[v][i];
+            if (v + 1 == kLiWaves || s_req[v + 1] != req) {
+                if (sum != 0u) atomicAdd(&p.histogram[static_cast<size_t>(req) * RPR * 256 + i], sum);
+                sum = 0;
             }
         }
     }
@@ -456,7 +497,10 @@ hipError_t launch_kernel(const KvipIndexerArgs& a, hipStream_t stream) {
         auto kernel = indexer_stream_kernel<ELEM, HEADS, RPR, W_BF16>;
         const int grid = stream_grid(kernel);
         if (grid == 0) return hipErrorInvalidDevice;
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLiThreads), 0, stream, a);
+        // No more workgroups than the block tables have tiles for (a page is a workgroup's four tiles).
+        const int64_t most = static_cast<int64_t>(a.batch) * a.max_blocks;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(std::min<int64_t>(grid, most))), dim3(kLiThreads), 0,
+                           stream, a);
     } else {
         const dim3 grid((a.max_blocks * kBlockTokens + kChunkTokens - 1) / kChunkTokens, a.batch);
         hipLaunchKernelGGL((indexer_chunk_kernel<ELEM, HEADS, RPR, W_BF16>), grid, dim3(kLiThreads), 0, stream, a);

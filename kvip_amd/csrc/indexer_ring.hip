@@ -5,13 +5,15 @@
 // wave of a grid that fills the GPU once takes one contiguous range of them (weighted by
 // dispatch round, see kRgLeadWeight). Each wave owns a 4-slot LDS ring (4 KiB of K rows +
 // 128 bytes of key scales per slot): direct-to-LDS loads (global_load_lds_dwordx4) bring
-// the next kRgDepth tiles while tile i is scored.
+// the next tile while tile i is scored (one: with ~2000 waves the HBM queues stay full, and
+// deeper rings only delay the first tiles of the workgroups dispatched last, whose waves then
+// finish last).
 // The loads apply the fragment swizzle on the global side (LDS row r, 16-byte slot s
 // holds piece s ^ (r & 7) of token r's row), so the MFMA B fragments are read straight
 // from the ring, bank-conflict free, with no transposition and no barrier (the ring is
-// private to the wave). The wave waits for its own loads with an exact vmcnt: every
-// iteration issues the same vector memory instructions (tiles past the range end repeat
-// its last tile into their own slot).
+// private to the wave). The wave waits for its own loads with an exact vmcnt. Nothing is
+// loaded past a range's last tile (a repeated tile per wave was 5 % of the traffic at 64 rows of
+// 8192-32768 tokens, and its wait ended every wave).
 //
 // Q fragments and per-lane head weights (w'_h = w_h * qscale_h) of the current request
 // stay in registers and are reloaded when the range crosses a request boundary. Scoring
@@ -20,8 +22,11 @@
 // half holds half of the heads of the tile's 32 tokens; after the per-lane-half head
 // reduction a v_permlane32_swap adds the other half's heads, and lanes 0-31 scale, round,
 // store the tile's keys and count them. The 256-bin high-byte histogram of the current
-// request is kept per wave in LDS (one buffer: a run covers one request) and added to the
-// global row at the run's end. LDS per workgroup stays under 80 KB so that two scoring
+// request is kept per wave in LDS and added to the global row when the wave's range crosses
+// into another request; what the waves of a workgroup hold at the end (mostly one request's) is
+// summed in LDS and added once per workgroup. Adds to one row serialise at ~10 ns each whoever
+// makes them, which bound few long rows when every wave added its own (one row of 32768
+// tokens: 16.2 us, now 7.8; of 131072: 29.0 us, now 11.9). LDS per workgroup stays under 80 KB so that two scoring
 // workgroups leave room on a CU for a 1024-thread TopK workgroup of another row group.
 //
 // Reference: QLIMatmul::ComputeMm1 (op_kernel/indexer/indexer_cube.h:161-322),
@@ -47,15 +52,15 @@ constexpr int kVmcntZero = 0x0F70;
 // Cache policy of the K-tile loads: nt (each index-K byte is read once per step; streamed
 // past the caches, reads run at ~7.0 TB/s on MI355X against ~6.3 TB/s with the default policy).
 constexpr int kNonTemporal = 2;
-// Tiles in flight per wave while one is scored (at most kRgSlots - 1). One: with ~2000
-// waves the HBM queues stay full, and deeper rings only delay the first tiles of the
-// workgroups dispatched last (their waves then finish last).
-constexpr int kRgDepth = 1;
 // Relative tile shares of the waves of the first dispatch round (the first workgroup on
 // each CU) and of the later rounds: the later workgroups' first tiles queue behind the
 // first round's and land ~2 us later at config-2 sizes, so they get ~18 % fewer tiles.
 constexpr int kRgLeadWeight = 22;
 constexpr int kRgLagWeight = 18;
+
+// Waves per request above which a workgroup adds its waves' histograms as one (1 us slower at 32
+// waves per row, where the adds are spread; 2 us faster at 256).
+constexpr int kRgCombineWaves = 128;
 
 // Stands in for a missing key-scale array (stride 0): 128 unit scales.
 __device__ __align__(16) float kRingUnitScale[kBlockTokens] = {
@@ -169,6 +174,7 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     __shared__ __align__(16) uint32_t s_hist[kRgWaves][256];
     __shared__ int s_prefix[kRgMaxBatch + 1];
     __shared__ uint32_t s_scan[kRgWaves];
+    __shared__ int s_req[kRgWaves];  // request of the histogram each wave still holds, -1: none
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -201,9 +207,18 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     const int64_t nw = static_cast<int64_t>(gridDim.x) * kRgWaves;
     const int64_t w = static_cast<int64_t>(blockIdx.x) * kRgWaves + wave;
     const int64_t weight_total = weight_before(nw);
-    int t = static_cast<int>(total_tiles * weight_before(w) / weight_total);
-    const int t_end = static_cast<int>(total_tiles * weight_before(w + 1) / weight_total);
-    if (t >= t_end) return;  // no barrier follows: waves run independently from here
+    int t, t_end;
+    if (total_tiles <= nw) {  // a tile per wave, packed into the first workgroups (fewer histogram adds)
+        t = static_cast<int>(w);
+        t_end = min(t + 1, total_tiles);
+        if (t - wave >= total_tiles) return;  // uniform for the workgroup
+    } else {
+        t = static_cast<int>(total_tiles * weight_before(w) / weight_total);
+        t_end = static_cast<int>(total_tiles * weight_before(w + 1) / weight_total);
+    }
+    // The waves run independently from here (to the barrier before the last histogram adds when the
+    // workgroup's are combined: with many waves per row; else the barrier costs more than it saves).
+    const bool combine = nw > kRgCombineWaves * p.batch;
 
     uint8_t* ring = &s_ring[wave][0][0];
     const uint32_t ring_lds = lds_addr(ring);
@@ -227,7 +242,8 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     const bool qscale = p.query_scale != nullptr;
     auto load_q = [&](int b) { rg_load_q<HEADS, W_BF16>(p, b, n, g, qscale, qa, wr); };
 
-    // The run's histogram (one request) in LDS, added to the global row at the run's end.
+    // The histogram in LDS (of one request) added to that request's global row, and cleared.
+    int held = -1;  // its request
     auto flush = [&](int req) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -265,10 +281,9 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
         const int next_b = __shfl_down(d_b, 1);
         const uint64_t run_ends = __ballot(lane < cnt && (lane == cnt - 1 || next_b != d_b));
 
-        auto issue = [&](int j) {
-            const int jj = min(j, cnt - 1);
-            const int page = __builtin_amdgcn_readlane(d_page, jj);
-            const int k = __builtin_amdgcn_readlane(d_k, jj);
+        auto issue = [&](int j) {  // j < cnt
+            const int page = __builtin_amdgcn_readlane(d_page, j);
+            const int k = __builtin_amdgcn_readlane(d_k, j);
             uint8_t* dst = ring + (j & (kRgSlots - 1)) * kRgSlotBytes;
             const uint8_t* src = kbase + static_cast<size_t>(page) * p.key_block_stride + (k & 3) * kRgTileBytes + src_lane;
 #pragma unroll
@@ -298,20 +313,19 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
         };
 
         // Q of the pass's first request is loaded ahead of the ring loads and waited for
-        // with them in flight (loads complete in order: at most the 15 ring-load
-        // instructions issued after it may remain).
+        // with them in flight (loads complete in order: at most the ring-load instructions
+        // issued after it may remain).
         const int b_first = __builtin_amdgcn_readlane(d_b, 0);
         if (b_first != qb) {
             load_q(b_first);
             qb = b_first;
         }
-#pragma unroll
-        for (int j = 0; j < kRgDepth; ++j) issue(j);
-        wait_vmcnt<kRgDepth * kRgOps>();
-        // Pipeline: loads of tiles i+1..i+kRgDepth stay in flight while tile i is scored.
-        // The vmcnt of each wait counts the vector memory instructions issued after tile
-        // i's loads (kRgDepth tile loads of kRgOps instructions plus the key stores in
-        // between); a Q reload or histogram flush in between only makes a wait longer.
+        issue(0);
+        wait_vmcnt<kRgOps>();
+        // Pipeline: the loads of tile i + 1 stay in flight while tile i is scored. The vmcnt of
+        // each wait counts the vector memory instructions issued after tile i's loads (the
+        // kRgOps of tile i + 1 and the key store of tile i - 1); a Q reload or histogram flush
+        // in between only makes a wait longer.
         int i = 0;
         while (i < cnt) {  // runs of one request
             const int b = __builtin_amdgcn_readlane(d_b, i);
@@ -322,26 +336,47 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
             }
             const uint64_t later = run_ends >> i;
             const int run_end = i + static_cast<int>(__builtin_ctzll(later)) + 1;
+            if (held >= 0 && held != b) flush(held);
+            held = b;
             for (; i < run_end; ++i) {
-                issue(i + kRgDepth);
-                if (i >= kRgDepth) {
-                    wait_vmcnt<kRgDepth * kRgOps + kRgDepth>();
-                } else if (i == 2) {
-                    wait_vmcnt<kRgDepth * kRgOps + 2>();
-                } else if (i == 1) {
-                    wait_vmcnt<kRgDepth * kRgOps + 1>();
+                if (i + 1 < cnt) {
+                    issue(i + 1);
+                    if (i >= 1) wait_vmcnt<kRgOps + 1>();
+                    else wait_vmcnt<kRgOps>();
+                } else if (i >= 1) {  // the pass's last tile: only the store before it may remain
+                    wait_vmcnt<1>();
                 } else {
-                    wait_vmcnt<kRgDepth * kRgOps>();
+                    wait_vmcnt<0>();
                 }
                 score(i);
             }
-            flush(b);
         }
-        wait_vmcnt<0>();  // repeated tail loads land before the ring is reused
         t += cnt;
+    }
+    if (!combine) {
+        if (held >= 0) flush(held);
+        report(p.status, err);
+        return;
+    }
+    // The held histograms, summed over consecutive waves of one request (the ranges are in
+    // order, so the requests are too). The adds above are not tracked by the compiler: waited here.
+    if (lane == 0) s_req[wave] = held;
+    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+    __syncthreads();
+    uint32_t sum = 0;
+#pragma unroll
+    for (int v = 0; v < kRgWaves; ++v) {
+        const int req = s_req[v];
+        if (req < 0) continue;  // uniform
+        sum += s_hist[v][tid];
+        if (v + 1 == kRgWaves || s_req[v + 1] != req) {
+            if (sum != 0u) atomicAdd(&p.histogram[static_cast<size_t>(req) * 256 + tid], sum);
+            sum = 0;
+        }
     }
     report(p.status, err);
 }
+static_assert(kRgThreads == 256, "one histogram bin per thread");
 
 // Keys of two 32-token tiles A and B for one query row: the same arithmetic as rg_key per
 // tile (MFMA over the heads, ReLU, head weights, four FMA chains per lane half in head
@@ -428,19 +463,17 @@ KVIP_DEVICE void lds_read_tile2(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t 
 // HBM once for all rows of its request; each wave keeps the Q fragments and weights of one
 // row in registers and finishes the keys of 64 tokens at once (lanes 0-31 the first 32,
 // lanes 32-63 the next 32: one key store and one histogram add per lane and tile).
-// Slots: kRrDepth tiles are in flight while tile i is scored, and the loads of tile
-// i + kRrDepth are issued while slow waves may still read tile i - 1, so the ring needs
-// kRrDepth + 2 slots (rounded up to a power of two; a full pass of kRgPass tiles then ends
-// on the last slot and the next pass starts on slot 0, away from the one still read).
+// Slots: one tile is in flight while tile i is scored, and the loads of tile i + 1 are issued
+// while slow waves may still read tile i - 1, so the ring needs three slots (four, a power of
+// two: a full pass of kRgPass tiles then ends on the last slot and the next pass starts on slot
+// 0, away from the one still read).
 // Every wave of a workgroup walks the same tiles, runs and passes, so all of them reach
 // the same barriers.
-constexpr int kRrDepth = 1;
-constexpr int kRrSlots = kRrDepth + 2 <= 4 ? 4 : 8;
+constexpr int kRrSlots = 4;
 constexpr int kRrTile = 64;                                // tokens per tile
 constexpr int kRrTileBytes = kRrTile * kIndexDim;          // 8 KiB of fp8 K rows
 constexpr int kRrSlotBytes = kRrTileBytes + kRrTile * 4;   // + 64 key scales
 static_assert(kRgPass % kRrSlots == 0, "a full pass ends on the last slot");
-static_assert(kRrDepth >= 1 && kRrDepth <= 4, "the waits below cover up to 4 tiles in flight");
 
 template <int ROWS, int HEADS, bool W_BF16>
 __global__ __launch_bounds__(ROWS * 64, 3) void indexer_rows_kernel(const KvipIndexerArgs p, int lead_blocks) {
@@ -547,11 +580,10 @@ __global__ __launch_bounds__(ROWS * 64, 3) void indexer_rows_kernel(const KvipIn
         const int next_b = __shfl_down(d_b, 1);
         const uint64_t run_ends = __ballot(lane < cnt && (lane == cnt - 1 || next_b != d_b));
 
-        // This wave's share of tile j's loads (tiles past the pass end repeat its last tile).
+        // This wave's share of tile j's loads (j < cnt).
         auto issue = [&](int j) {
-            const int jj = min(j, cnt - 1);
-            const int page = __builtin_amdgcn_readlane(d_page, jj);
-            const int k = __builtin_amdgcn_readlane(d_k, jj);
+            const int page = __builtin_amdgcn_readlane(d_page, j);
+            const int k = __builtin_amdgcn_readlane(d_k, j);
             uint8_t* dst = ring + (j & (kRrSlots - 1)) * kRrSlotBytes;
             const uint8_t* src = kbase + static_cast<size_t>(page) * p.key_block_stride + (k & 1) * kRrTileBytes + src_lane;
 #pragma unroll
@@ -585,8 +617,7 @@ __global__ __launch_bounds__(ROWS * 64, 3) void indexer_rows_kernel(const KvipIn
             rg_load_q<HEADS, W_BF16>(p, b_first * ROWS + wave, n, g, qscale, qa, wr);
             qb = b_first;
         }
-#pragma unroll
-        for (int j = 0; j < kRrDepth; ++j) issue(j);
+        issue(0);
         int i = 0;
         while (i < cnt) {  // runs of one request
             const int b = __builtin_amdgcn_readlane(d_b, i);
@@ -598,26 +629,22 @@ __global__ __launch_bounds__(ROWS * 64, 3) void indexer_rows_kernel(const KvipIn
             const uint64_t later = run_ends >> i;
             const int run_end = i + static_cast<int>(__builtin_ctzll(later)) + 1;
             for (; i < run_end; ++i) {
-                issue(i + kRrDepth);
-                // Own share of tile i landed: after its loads come those of the next
-                // kRrDepth tiles and the key stores of the (at most kRrDepth) tiles before i.
-                if (i >= kRrDepth) {
-                    wait_vmcnt<kRrDepth * kOps + kRrDepth>();
-                } else if (kRrDepth > 3 && i == 3) {
-                    wait_vmcnt<kRrDepth * kOps + (kRrDepth > 3 ? 3 : 0)>();
-                } else if (kRrDepth > 2 && i == 2) {
-                    wait_vmcnt<kRrDepth * kOps + (kRrDepth > 2 ? 2 : 0)>();
-                } else if (kRrDepth > 1 && i == 1) {
-                    wait_vmcnt<kRrDepth * kOps + (kRrDepth > 1 ? 1 : 0)>();
+                // Own share of tile i landed: after its loads come those of tile i + 1 (none at the
+                // pass's end) and the key store of tile i - 1.
+                if (i + 1 < cnt) {
+                    issue(i + 1);
+                    if (i >= 1) wait_vmcnt<kOps + 1>();
+                    else wait_vmcnt<kOps>();
+                } else if (i >= 1) {
+                    wait_vmcnt<1>();
                 } else {
-                    wait_vmcnt<kRrDepth * kOps>();
+                    wait_vmcnt<0>();
                 }
                 __builtin_amdgcn_s_barrier();  // every wave's share of tile i landed
                 score(i);
             }
             flush(b * ROWS + wave);
         }
-        wait_vmcnt<0>();  // the repeated tail load lands before the ring is reused
         t += cnt;
     }
     report(p.status, err);
@@ -650,7 +677,10 @@ hipError_t launch_ring_kernel(const KvipIndexerArgs& a, int tile_lo, int tile_hi
     auto kernel = indexer_ring_kernel<HEADS, W_BF16>;
     const RingGrid grid = ring_grid(kernel);
     if (grid.blocks == 0) return hipErrorInvalidDevice;
-    hipLaunchKernelGGL(kernel, dim3(grid.blocks), dim3(kRgThreads), 0, stream, a, grid.lead_blocks, tile_lo, tile_hi);
+    // No more workgroups than the block tables have tiles for (one page is one workgroup's four tiles).
+    const int64_t most = static_cast<int64_t>(a.batch) * a.max_blocks;
+    const int blocks = static_cast<int>(most < grid.blocks ? most : grid.blocks);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kRgThreads), 0, stream, a, grid.lead_blocks, tile_lo, tile_hi);
     return hipGetLastError();
 }
 
