@@ -3,10 +3,10 @@
 // memset), so the whole round can be captured into a single hipGraph. The default plan is
 // three launches: scoring (indexer_ring.hip), TopK with the row's keys in registers
 // (topk.hip; rows above 65536 keys take the multi-workgroup split select) and the
-// gather (fetch_gather.hip). Measured at config 2 this beats TopK fused with the
-// gather (select_fetch.hip, still exported as kvip_hip_select_fetch): the separate gather
-// launch is balanced by the hardware dispatcher, while the fused one waits for its
-// slowest workgroup.
+// gather (fetch_gather.hip). At config 2 this beats TopK fused with the gather (select_fetch.hip):
+// the separate gather launch is balanced by the hardware dispatcher, while the fused one waits
+// for its slowest workgroup. Up to kFusedRows query rows leave most of the chip idle in either
+// launch, and the fused one wins by the second launch's latencies (figures in select_fetch.hip).
 //
 // Replaces kvip_lifetch_streaming_forward (csrc/operators/lightning_indexer_with_fetch/
 // include/api.h:7, op_host/launch.cpp:76-83), whose init -> LI -> resolve/update/fetch
@@ -20,11 +20,15 @@ uint32_t validate_fetch(const KvipFetchArgs* a);
 hipError_t launch_indexer(const KvipIndexerArgs& a, hipStream_t stream);
 hipError_t launch_topk(const KvipTopkArgs& a, hipStream_t stream);
 hipError_t launch_fetch(const KvipFetchArgs& a, hipStream_t stream);
+uint32_t validate_select_fetch(const KvipTopkArgs* t, const KvipFetchArgs* f);
+hipError_t launch_select_fetch(const KvipTopkArgs& t, const KvipFetchArgs& f, hipStream_t stream);
 }  // namespace kvip
 
 extern "C" uint32_t kvip_hip_abi_version(void) { return KVIP_HIP_ABI_VERSION; }
 
 namespace {
+constexpr int kFusedRows = 16;  // 16 rows 1 us faster fused, 24 rows 1 us slower
+
 // Validates the chained arguments and picks the launch plan (KVIP_LIFETCH_PLAN_*), or
 // returns KVIP_ERR_INVALID.
 uint32_t lifetch_plan(const KvipLIFetchArgs* args) {
@@ -58,6 +62,10 @@ extern "C" uint32_t kvip_hip_lifetch_forward(const KvipLIFetchArgs* args, void* 
     const KvipFetchArgs& fe = args->fetch;
     hipError_t e = kvip::launch_indexer(li, s);
     if (e != hipSuccess) return static_cast<uint32_t>(e);
+    // Few query rows: TopK fused with the gather (needs the work memory's tickets).
+    if (li.batch * li.rows_per_request <= kFusedRows && kvip::validate_select_fetch(&tk, &fe) == KVIP_OK) {
+        return static_cast<uint32_t>(kvip::launch_select_fetch(tk, fe, s));
+    }
     // Rows that fit the register-resident TopK take it even when the split select's work
     // memory is given.
     KvipTopkArgs t = tk;

@@ -435,3 +435,36 @@ def test_select_fetch_rejects_rows_beyond_32768_and_forward_falls_back(torch_gpu
         assert np.array_equal(topk[r], ref.topk_reference(keys[r], v))
     assert np.array_equal(upd.output.cpu().numpy(),
                           ref.fetch_gather(wl.kv_cache.cpu().numpy(), wl.block_table.cpu().numpy(), topk))
+
+
+@pytest.mark.parametrize("qk", ["fp8", "bf16"])
+@pytest.mark.parametrize("batch,rpr,ctx_low,ctx_high", [
+    (1, 1, 2048, 2048), (1, 1, 2047, 2047), (1, 1, 8192, 8192), (1, 1, 32768, 32768), (1, 4, 8193, 8200),
+    (3, 1, 1, 16385), (5, 2, 100, 4000), (16, 1, 2000, 9000), (17, 1, 2000, 9000), (2, 1, 32769, 70000)])
+def test_forward_of_few_rows_equals_its_stages(torch_gpu, qk, batch, rpr, ctx_low, ctx_high):
+    """The forward (TopK fused with the gather up to 16 query rows of 32768 keys, the three
+    launches above) against scoring, TopK and gather launched one by one: the same TopK and
+    rows bit for bit, the histograms and counters back at zero, three times in a row."""
+    torch = torch_gpu
+    say(f"case few rows {qk} batch={batch} rpr={rpr} ctx={ctx_low}..{ctx_high}")
+    wl = synthetic.decode_workload(torch, batch=batch, ctx_low=ctx_low, ctx_high=ctx_high, device="cuda", qk=qk,
+                                   key_scale=qk == "fp8", rows_per_request=rpr, seed=batch + ctx_high,
+                                   max_context=ctx_high)
+    ends = np.maximum(np.repeat(wl.ctx, rpr) - rpr + 1 + np.tile(np.arange(rpr), batch), 0)
+    rot, upd, fwd = synthetic.bind(torch, kvip_amd, wl, query_ends=ends)
+    fwd.score()
+    totals = rot.histogram.sum(1).cpu().numpy()
+    assert np.array_equal(totals, ends)  # every visible key counted once
+    fwd.select()
+    fwd.fetch()
+    topk, rows = rot.topk.clone(), upd.output.clone()
+    assert torch.equal(rot.topk.cpu(), torch.from_numpy(np.stack(
+        [ref.topk_reference(k, int(v)) for k, v in zip(gpu_keys(rot), ends)])))
+    for attempt in range(3):
+        rot.topk.fill_(-5)
+        upd.output.fill_(0xAB)
+        fwd()
+        torch.cuda.synchronize()
+        assert int(rot.status.item()) == 0
+        assert torch.equal(rot.topk, topk) and torch.equal(upd.output, rows), attempt
+        assert not rot.histogram.any() and not rot.topk_segments[:, 0, -1].any()
