@@ -15,31 +15,33 @@ namespace kvip {
 namespace {
 
 constexpr int kGatherThreads = 256;
-constexpr int kRowsPerWave = 32;
-constexpr int kRowsPerBlock = kRowsPerWave * (kGatherThreads / 64);
+constexpr int kWaves = kGatherThreads / 64;
+// Rows per wave: 32, or 16 up to kFewSelections, which leave CUs idle (8 query rows: 8.6 -> 6.5 us,
+// 24: 14.2 -> 12.6, 32: 16.2 and 16.3, 64: 30.5 -> 32.3; 8 rows per wave are slower from 8 query rows).
+constexpr uint32_t kFewSelections = 24 * kTopK;
 // Outputs above this size are stored with the nontemporal policy: they do not fit the
 // 256 MB memory-side cache, so caching the stream only evicts lines the gather still reads
 // (4-row MTP decode, 344 MB: 145 -> 141 us); smaller outputs (config 2, 86 MB) stay
 // cached, where the default policy is 3 us faster.
 constexpr uint64_t kStreamOutputBytes = 192ull << 20;
 
-// One wave moves 32 consecutive selected rows: lanes 0..31 translate the token ids to
+// One wave moves ROWS consecutive selected rows: lanes 0..ROWS-1 translate the token ids to
 // source rows (token id -> block table -> byte offset), then all 64 lanes copy the
-// 32*PIECES 16-byte pieces (21 loads in flight per lane for 656-byte rows). Because the
+// ROWS*PIECES 16-byte pieces (32 rows: 21 loads in flight per lane for 656-byte rows). Because the
 // destination rows are consecutive, the wave's output
 // is one contiguous range written with fully coalesced 16-byte stores.
-template <int PIECES, bool NT_STORE>
+template <int ROWS, int PIECES, bool NT_STORE>
 __global__ __launch_bounds__(kGatherThreads) void fetch_gather_kernel(const KvipFetchArgs p, uint32_t selections) {
     const int pieces = PIECES > 0 ? PIECES : p.row_bytes / 16;
     const int lane = threadIdx.x & 63;
     uint32_t err = 0;
-    const uint32_t sel0 = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) * kRowsPerWave;
+    const uint32_t sel0 = blockIdx.x * (ROWS * kWaves) + (threadIdx.x >> 6) * ROWS;
     if (sel0 >= selections) return;
     const int capacity = p.max_blocks * kBlockTokens;
 
     // Source byte offset of row (sel0 + lane), or -1 for an empty / invalid entry.
     int64_t src = -1;
-    if (lane < kRowsPerWave && sel0 + lane < selections) {
+    if (lane < ROWS && sel0 + lane < selections) {
         const uint32_t sel = sel0 + lane;
         const int t = p.topk[sel];
         const int b = static_cast<int>(sel / kTopK) / p.rows_per_request;
@@ -54,10 +56,10 @@ __global__ __launch_bounds__(kGatherThreads) void fetch_gather_kernel(const Kvip
             }
         }
     }
-    const int rows = min(kRowsPerWave, static_cast<int>(selections - sel0));
+    const int rows = min(ROWS, static_cast<int>(selections - sel0));
     const int total = rows * pieces;
     uint8_t* dst = p.output + static_cast<size_t>(sel0) * p.row_bytes;
-    constexpr int kMaxIters = PIECES > 0 ? (kRowsPerWave * PIECES + 63) / 64 : 1;
+    constexpr int kMaxIters = PIECES > 0 ? (ROWS * PIECES + 63) / 64 : 1;
     if constexpr (PIECES > 0) {
         v4i val[kMaxIters];
 #pragma unroll
@@ -65,7 +67,7 @@ __global__ __launch_bounds__(kGatherThreads) void fetch_gather_kernel(const Kvip
             const int idx = it * 64 + lane;
             const int r = idx / PIECES;
             const int piece = idx - r * PIECES;
-            const int64_t base = row_value<PIECES, kRowsPerWave>(src, it, r);
+            const int64_t base = row_value<PIECES, ROWS>(src, it, r);
             val[it] = v4i{0, 0, 0, 0};
             if (idx < total && base >= 0) {
                 val[it] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(p.kv_cache + base + piece * 16));
@@ -83,12 +85,12 @@ __global__ __launch_bounds__(kGatherThreads) void fetch_gather_kernel(const Kvip
             }
         }
     } else {
-        const int iters = (kRowsPerWave * pieces + 63) / 64;  // uniform: every lane joins each shuffle
+        const int iters = (ROWS * pieces + 63) / 64;  // uniform: every lane joins each shuffle
         for (int it = 0; it < iters; ++it) {
             const int idx = it * 64 + lane;
             const int r = idx / pieces;
             const int piece = idx - r * pieces;
-            const int64_t base = __shfl(src, min(r, kRowsPerWave - 1));
+            const int64_t base = __shfl(src, min(r, ROWS - 1));
             v4i v = v4i{0, 0, 0, 0};
             if (idx < total && base >= 0) v = *reinterpret_cast<const v4i*>(p.kv_cache + base + piece * 16);
             if (idx < total) *reinterpret_cast<v4i*>(dst + static_cast<size_t>(idx) * 16) = v;
@@ -115,20 +117,26 @@ uint32_t validate_fetch(const KvipFetchArgs* a) {
     return ok ? KVIP_OK : KVIP_ERR_INVALID;
 }
 
+namespace {
+template <int ROWS, int PIECES, bool NT_STORE>
+void launch_rows(const KvipFetchArgs& a, uint32_t selections, hipStream_t stream) {
+    constexpr uint32_t per_block = ROWS * kWaves;
+    hipLaunchKernelGGL((fetch_gather_kernel<ROWS, PIECES, NT_STORE>), dim3((selections + per_block - 1) / per_block),
+                       dim3(kGatherThreads), 0, stream, a, selections);
+}
+}  // namespace
+
 hipError_t launch_fetch(const KvipFetchArgs& a, hipStream_t stream) {
     const uint32_t selections = static_cast<uint32_t>(a.batch) * a.rows_per_request * kTopK;
-    const dim3 grid((selections + kRowsPerBlock - 1) / kRowsPerBlock);
     const bool stream_out = static_cast<uint64_t>(selections) * a.row_bytes > kStreamOutputBytes;
-    if (a.row_bytes == KVIP_KV_ROW_BYTES) {
-        if (stream_out) {
-            hipLaunchKernelGGL((fetch_gather_kernel<KVIP_KV_ROW_BYTES / 16, true>), grid, dim3(kGatherThreads), 0,
-                               stream, a, selections);
-        } else {
-            hipLaunchKernelGGL((fetch_gather_kernel<KVIP_KV_ROW_BYTES / 16, false>), grid, dim3(kGatherThreads), 0,
-                               stream, a, selections);
-        }
+    if (a.row_bytes != KVIP_KV_ROW_BYTES) {
+        launch_rows<32, 0, false>(a, selections, stream);
+    } else if (stream_out) {
+        launch_rows<32, KVIP_KV_ROW_BYTES / 16, true>(a, selections, stream);
+    } else if (selections <= kFewSelections) {
+        launch_rows<16, KVIP_KV_ROW_BYTES / 16, false>(a, selections, stream);
     } else {
-        hipLaunchKernelGGL((fetch_gather_kernel<0, false>), grid, dim3(kGatherThreads), 0, stream, a, selections);
+        launch_rows<32, KVIP_KV_ROW_BYTES / 16, false>(a, selections, stream);
     }
     return hipGetLastError();
 }

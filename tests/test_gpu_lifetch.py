@@ -468,3 +468,33 @@ def test_forward_of_few_rows_equals_its_stages(torch_gpu, qk, batch, rpr, ctx_lo
         assert int(rot.status.item()) == 0
         assert torch.equal(rot.topk, topk) and torch.equal(upd.output, rows), attempt
         assert not rot.histogram.any() and not rot.topk_segments[:, 0, -1].any()
+
+
+@pytest.mark.parametrize("kind,ctx", [
+    ("random", [131072, 65537, 73728, 73729, 2047, 0, 2048]),
+    ("few_levels", [100000, 8193]),
+    ("all_equal", [70000, 65536, 16384]),
+    ("one_bin", [81921, 131071]),
+])
+def test_topk_of_long_rows_on_wide_segments(torch_gpu, kind, ctx):
+    """The split select of rows above 65536 keys (8192-key segments of 1024 threads): rows that end on
+    a segment, one key past it and far before the stride, ties across segments; the work
+    memory's last word of a row's first record stays zero."""
+    torch = torch_gpu
+    say(f"case wide split {kind} {ctx}")
+    rng = np.random.default_rng(len(ctx) * 11 + ctx[0])
+    rot = kvip_amd.LIFetchBinding(torch, batch=len(ctx), max_context=max(ctx), device="cuda")
+    keys = np.zeros((len(ctx), rot.key_stride), np.uint16)
+    for r, v in enumerate(ctx):
+        keys[r, :v] = keys_case(kind, v, rng)
+    hist = np.stack([np.bincount(keys[r, :v] >> 8, minlength=256) for r, v in enumerate(ctx)])
+    rot.score_keys.copy_(torch.from_numpy(keys.view(np.int16)))
+    rot.seq_lens.copy_(torch.tensor(ctx, dtype=torch.int32))
+    for attempt in range(2):
+        rot.histogram.copy_(torch.from_numpy(hist.astype(np.int32)))
+        rot.topk.fill_(-5)
+        got = run_topk(torch, rot, use_histogram=True)
+        for r, v in enumerate(ctx):
+            assert np.array_equal(got[r], ref.topk_reference(keys[r], v)), f"row {r} valid {v}"
+        assert int(rot.status.item()) == 0
+        assert not rot.histogram.any() and not rot.topk_segments[:, 0, -1].any()
