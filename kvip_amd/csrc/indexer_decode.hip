@@ -146,7 +146,7 @@ struct Tile {
         // Add the other lane half's heads (v_permlane32_swap: lane l <-> lane l^32).
         const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_int(part), __float_as_int(part), false, false);
         part += __int_as_float(g == 0 ? swapped[1] : swapped[0]);
-        return sortable_key(bf16_bits_half_away(part * ks));
+        return score_key(part * ks);
     }
 };
 

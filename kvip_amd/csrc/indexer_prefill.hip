@@ -7,8 +7,8 @@
 // stride over the units, kvip_hip_indexer_prefill_grid). fp8: 4 waves own 2 query rows
 // each; bf16 (Q fragments twice as large): 8 waves own one row each. A wave keeps its rows'
 // Q fragments and per-lane head weights (w'_h = w_h * qscale_h for the 32 heads a lane
-// reduces) in registers. The segment streams through LDS in 32 KiB chunks (256 fp8 or 128
-// bf16 tokens), double buffered: every wave issues direct-to-LDS 16-byte loads
+// reduces) in registers. The segment streams through LDS in chunks of 256 tokens (fp8 32 KiB,
+// bf16 64 KiB), double buffered: every wave issues direct-to-LDS 16-byte loads
 // (global_load_lds_dwordx4) for its share of the next chunk, with the XOR swizzle applied
 // on the global side so that the fragment reads (lane n of a 32-token tile reads row n)
 // hit distinct bank groups. Each chunk tile (32 tokens) is one B fragment set read once
@@ -20,6 +20,19 @@
 // per word: bins b and b + 128; bf16, whose 64 lanes add to one row, keeps four copies per
 // row) is added to the row histograms at the end. fp8 runs two workgroups per CU, bf16 one
 // (two waves per SIMD either way).
+//
+// Bound: matrix cores and VALU together, under the card's power limit. A 32-token tile of one fp8
+// row with 64 heads is 256 cycles of MFMA and 64 VALU operations (ReLU and weight FMA). A loop of
+// just these takes 190-197 ns per tile with two waves per SIMD and 186 ns with three or four; its
+// MFMAs alone take 149 ns, at the 1.7 GHz that they leave on random data. This kernel takes about
+// 235 ns, with its staging, LDS reads, the finish of each tile and the histogram. The order of MFMA
+// and VALU operations within a tile moves it by less than 3%; one fp8 row per wave at four waves
+// per SIMD spills and is twice as slow. What could be trimmed is around the loop: both rows (bf16:
+// both tiles) are joined by one lane swap, the key comes straight from the rounded 32-bit pattern,
+// the next tile's fragments are requested under the epilogue, and bf16 chunks are as long as fp8
+// ones, with half the barriers they had at 128 tokens. Scoring 4096 rows causally against 65536
+// keys in fp8 went from 1948 to 1905 us, six sequences of up to 900 rows against up to 9000 keys
+// from 150 to 142 us, 2048 rows against 16384 keys in bf16 from 462 to 454 us.
 //
 // Reference: the native prefill LI (torch_npu.npu_quant_lightning_indexer, TND layout,
 // sparse_mode 3) that the vLLM selector runs for prefill rows (python/kvip/adapters/vllm/
@@ -44,7 +57,6 @@ struct PfShape {
     static constexpr int kRows = kPfBlockRows / kWaves;
     static constexpr int kThreads = kWaves * 64;
 };
-constexpr int kPfChunkBytes = 256 * kIndexDim;             // 32 KiB of K rows per LDS chunk
 constexpr int kPfSegment = 4096;                            // key positions per workgroup
 constexpr int kPfPages = kPfSegment / kBlockTokens;         // 32
 constexpr int kPfMaxSeq = KVIP_PREFILL_MAX_SEQUENCES;
@@ -66,11 +78,20 @@ KVIP_DEVICE float pf_weight(const KvipPrefillArgs& p, size_t idx) {
     return w * (p.query_scale != nullptr ? p.query_scale[idx] : 1.0f);
 }
 
+// Counts a key's high byte in a row histogram of two 16-bit counters per word: bins b and
+// b ^ 128 share a word (the populated bins of a row are adjacent and would otherwise serialise
+// on one word's atomics).
+KVIP_DEVICE void pf_count(uint32_t hist, uint32_t key) {
+    __hip_atomic_fetch_add((LdsU32)(hist + ((key >> 6) & 0x1FCu)), key & 0x8000u ? 0x10000u : 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 template <int ELEM, int HEADS, bool W_BF16>
 __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_prefill_kernel(const KvipPrefillArgs p) {
     constexpr int kPfWaves = PfShape<ELEM>::kWaves;
     constexpr int kPfRowsPerWave = PfShape<ELEM>::kRows;
     constexpr int kPfThreads = PfShape<ELEM>::kThreads;
+    constexpr int kPfChunkBytes = 256 * kIndexDim * ELEM;  // 256 tokens per LDS chunk
     constexpr int MT = HEADS / 32;
     constexpr int NV = Mma<ELEM>::NV;              // 16-byte pieces of a half row per lane
     constexpr int STEPS = Mma<ELEM>::STEPS;        // MFMAs per 128-dim contraction
@@ -193,11 +214,13 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
         my_ok = ok ? 1.0f : 0.0f;
         if (!ok) err |= KVIP_STATUS_BAD_BLOCK;
     }
+    const bool pages_ok = __ballot(lane < kPfPages && my_ok == 0.0f) == 0ull;  // uniform
     const uint8_t* kbase = static_cast<const uint8_t*>(p.keys);
 
     // Wave w stages rows [w * chunk/4, (w + 1) * chunk/4) of a chunk (one page's rows):
     // 8 direct-to-LDS loads of kRowsPerLoad rows each.
     constexpr int kWaveRows = kPfChunk / kPfWaves;
+    const uint32_t k_lds = lds_addr(&s_k[0][0]), ks_lds = lds_addr(&s_ks[0][0]);
     auto stage = [&](int c, int buf) {
         const int pg = __builtin_amdgcn_readlane(my_page, c * kChunkPages + (wave * kWaveRows) / kBlockTokens);
 #pragma unroll
@@ -206,8 +229,7 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
             const int piece = (lane % kPieces) ^ pf_swizzle<ELEM>(row);
             const uint8_t* src = kbase + static_cast<size_t>(pg) * p.key_block_stride +
                                  (row & (kBlockTokens - 1)) * kRowBytes + piece * 16;
-            __builtin_amdgcn_global_load_lds(src, LDS_PTR(&s_k[buf][(wave * kWaveRows + v * kRowsPerLoad) * kRowBytes]),
-                                             16, 0, 0);
+            dma16(src, k_lds + buf * kPfChunkBytes + (wave * kWaveRows + v * kRowsPerLoad) * kRowBytes);
         }
         if (wave == 0 && p.key_scale != nullptr && lane < kPfChunk / 4) {
             const int row = lane * 4;  // 4 consecutive scales of one page
@@ -216,7 +238,7 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
             const int pg1 = __builtin_amdgcn_readlane(my_page, c * kChunkPages + kChunkPages - 1);
             const int pg = lane < 32 ? pg0 : pg1;
             const float* src = p.key_scale + static_cast<size_t>(pg) * p.scale_block_stride + (row & 127);
-            __builtin_amdgcn_global_load_lds(src, LDS_PTR(&s_ks[buf][0]), 16, 0, 0);
+            dma16(reinterpret_cast<const uint8_t*>(src), ks_lds + buf * kPfChunk * 4);
         }
     };
     if (p.key_scale == nullptr) {  // unit key scales, written once before the loop
@@ -224,23 +246,21 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
         __syncthreads();
     }
 
-    // This lane half's row (one row per wave: the row of both halves; its keys and
-    // histogram come from lanes 0-31).
+    // This lane half's row (one row per wave: the row of both halves).
     int vis_mine, vis_max_wave;
     if constexpr (kPfRowsPerWave == 2) {
         vis_mine = g == 0 ? vis[0] : vis[1];
         vis_max_wave = max(vis[0], vis[1]);
     } else {
-        vis_mine = g == 0 ? vis[0] : 0;
+        vis_mine = vis[0] - 32 * g;  // lane half g finishes tile k + g
         vis_max_wave = vis[0];
     }
     const int hist_row = wave * kPfRowsPerWave + (kPfRowsPerWave == 2 ? g : 0);
-    // Per-lane LDS addresses: the tile row's four swizzled K pieces (the swizzle of row
-    // k*32 + n does not depend on k), its key scale, and the key strip slots.
-    uint32_t ka[NV];
-#pragma unroll
-    for (int u = 0; u < NV; ++u) ka[u] = lds_addr(&s_k[0][n * kRowBytes + (((g * NV + u) ^ pf_swizzle<ELEM>(n)) * 16)]);
-    const uint32_t ksa = lds_addr(&s_ks[0][n]);
+    // Per-lane LDS addresses: the tile row's first swizzled K piece (the swizzle of row k*32 + n
+    // does not depend on k; piece u sits at the address XOR 16 u), its key scale, and the key strip
+    // slots.
+    const uint32_t ka = k_lds + n * kRowBytes + (((g * NV) ^ pf_swizzle<ELEM>(n)) * 16);
+    const uint32_t ksa = ks_lds + n * 4;
     const uint32_t keya = lds_addr(&s_keys[wave][kPfRowsPerWave == 2 ? g : 0][n]);
     const uint32_t hista = lds_addr(&s_hist[hist_row][(lane % kHistCopies) * kHistStride]);
     constexpr uint32_t kKBuf = kPfChunkBytes;          // bytes between the two K buffers
@@ -253,162 +273,146 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
         lds_barrier(stores);  // chunk c landed and is visible; buffer c+1 is free again
         if (c + 1 < nchunks) stage(c + 1, buf ^ 1);
         const int cstart = seg0 + c * kPfChunk;
+        // A lane's key of tile k is visible while 32 k is below this.
+        const int left = vis_mine - cstart - n;
         const float page_ok0 =
             __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_ok), c * kChunkPages));
         const float page_ok1 = __builtin_bit_cast(
             float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, my_ok), c * kChunkPages + kChunkPages - 1));
+        // Tile k's fragments and key scale. They are requested as soon as the MFMAs of the tile before
+        // are issued, so that the reads pass under that tile's epilogue; the chunk's last tile repeats
+        // its own.
+        auto load_tile = [&](int k, v4i (&kb)[NV], float& ks) {
+            const uint32_t a = ka + buf * kKBuf + k * 32 * kRowBytes;
+#pragma unroll
+            for (int u = 0; u < NV; ++u) kb[u] = *(LdsV4i)(a ^ (u * 16));
+            ks = *(LdsF32)(ksa + buf * kSBuf + k * 128);
+        };
         if constexpr (kPfRowsPerWave == 1) {
             // One row per wave (bf16): two tiles per step, finished together. Lane half g
             // finishes tile k + g: one lane-half swap joins both tiles' head halves, so every
             // lane stores a key and counts it (the same sums, in the same order, as one tile
             // at a time).
+            v4i kb[NV];
+            float ks_raw[2];
+            load_tile(0, kb, ks_raw[0]);
 #pragma unroll 1
             for (int k = 0; k < kPfTiles; k += 2) {
                 const int t0 = cstart + k * 32;
                 if (t0 >= vis_max_wave) break;  // uniform per wave: later tiles are masked too
-                float part2[2];
-                float ks = 0.f;
+                float pj[2][4], ks;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const int kt = k + h;
-                    v4i kb[NV];
-                    float ks_raw;
-                    const uint32_t toff = buf * kKBuf + kt * 32 * kRowBytes;
-                    lds_read_tile8(ka, toff, ksa + buf * kSBuf + kt * 128, kb, ks_raw);
-                    if (g == h) ks = ks_raw * (kt < kPfTiles / 2 ? page_ok0 : page_ok1);
-                // Units u = (row q = u / MT, head tile mt = u % MT), two dependent K-slice MFMAs
-                // each. Unit u+1's MFMAs are issued between the 32 VALU ops (ReLU, weight FMA) of
-                // unit u's epilogue so that the matrix core and the VALU work side by side.
-                constexpr int U = kPfRowsPerWave * MT;
-                float pj[kPfRowsPerWave][4];
+                    pj[h][0] = pj[h][1] = pj[h][2] = pj[h][3] = 0.f;
+                    if (h == 0 || g == 1) ks = ks_raw[h];
+                    // As below, with head tiles of STEPS MFMAs each: head tile u + 1's MFMAs are issued
+                    // between the 32 VALU ops of head tile u.
+                    v16f acc[2];
 #pragma unroll
-                for (int q = 0; q < kPfRowsPerWave; ++q) pj[q][0] = pj[q][1] = pj[q][2] = pj[q][3] = 0.f;
-                v16f acc[2];
-                acc[0] = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                    for (int u = -1; u < MT; ++u) {  // step -1: head tile 0's MFMAs
+                        v16f& nxt = acc[(u + 1) & 1];
+                        if (u + 1 < MT) {
+                            nxt = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int st = 0; st < STEPS; ++st) Mma<ELEM>::step(st, qa[0][0], kb, acc[0]);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int q = u / MT, mt = u % MT;
-                    v16f& cur = acc[u & 1];
-                    v16f& nxt = acc[(u + 1) & 1];
-                    if (u + 1 < U) {
-                        nxt = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int st = 0; st < STEPS; ++st) Mma<ELEM>::step(st, qa[(u + 1) / MT][(u + 1) % MT], kb, nxt);
-                    }
-#pragma unroll
-                    for (int r4 = 0; r4 < 4; ++r4) {
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                                const float relu = __int_as_float(max(__float_as_int(cur[r4 * 4 + j]), 0));
-                                pj[q][j] = fmaf(relu, wr[q][mt * 16 + r4 * 4 + j], pj[q][j]);
+                            for (int st = 0; st < STEPS; ++st) Mma<ELEM>::step(st, qa[0][u + 1], kb, nxt);
                         }
-                    }
-                    if (u + 1 < U) {
-                        // The next unit's STEPS MFMAs spread over this unit's 32 VALU ops (fp8:
-                        // 1 MFMA, 16 VALU, 1 MFMA, 16 VALU; bf16: 1 MFMA, 4 VALU, ...); nothing
-                        // crosses into the next unit.
+                        if (u >= 0) {
+                            const v16f& cur = acc[u & 1];
 #pragma unroll
-                        for (int st = 0; st < STEPS; ++st) {
+                            for (int r4 = 0; r4 < 4; ++r4) {
+#pragma unroll
+                                for (int j = 0; j < 4; ++j) {
+                                    const float relu = __int_as_float(max(__float_as_int(cur[r4 * 4 + j]), 0));
+                                    pj[h][j] = fmaf(relu, wr[0][u * 16 + r4 * 4 + j], pj[h][j]);
+                                }
+                            }
+                        }
+                        if (u >= 0 && u + 1 < MT) {
+#pragma unroll
+                            for (int st = 0; st < STEPS; ++st) {
                                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                                 __builtin_amdgcn_sched_group_barrier(0x002, 32 / STEPS, 0);
+                            }
                         }
-                        __builtin_amdgcn_sched_barrier(0);
+                        if (u + 1 < MT) __builtin_amdgcn_sched_barrier(0);
+                        if (u + 2 == MT) {  // the tile's last MFMAs are issued
+                            load_tile(min(k + h + 1, kPfTiles - 1), kb, ks_raw[1 - h]);
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
                     }
                 }
-                    part2[h] = (pj[0][0] + pj[0][1]) + (pj[0][2] + pj[0][3]);
-                }
+                if (!pages_ok) ks *= k + g < kPfTiles / 2 ? page_ok0 : page_ok1;
+                const float part0 = (pj[0][0] + pj[0][1]) + (pj[0][2] + pj[0][3]);
+                const float part1 = (pj[1][0] + pj[1][1]) + (pj[1][2] + pj[1][3]);
                 // [tile k lanes 0-31, tile k + 1 lanes 0-31] + [tile k lanes 32-63, tile k + 1 lanes 32-63].
-                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(part2[0]), __float_as_int(part2[1]),
-                                                                 false, false);
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(part0), __float_as_int(part1), false, false);
                 const float total = __int_as_float(sw[0]) + __int_as_float(sw[1]);
-                const uint32_t key = sortable_key(bf16_bits_half_away(total * ks));
-                lds_write_b16(keya + (k + g) * 64, key);
-                if (t0 + 32 * g + n < vis[0]) {
-                    const uint32_t bin = key >> 8;
-                    lds_add_u32(hista + (bin & 127) * 4, 1u << (16 * (bin >> 7)));
-                }
+                const uint32_t key = score_key(total * ks);
+                *(LdsU16)(keya + (k + g) * 64) = static_cast<uint16_t>(key);
+                if (k * 32 < left) pf_count(hista, key);
             }
         } else {
-    #pragma unroll 1
+            v4i kb[NV];
+            float ks_raw;
+            load_tile(0, kb, ks_raw);
+#pragma unroll 1
             for (int k = 0; k < kPfTiles; ++k) {
                 const int t0 = cstart + k * 32;
                 if (t0 >= vis_max_wave) break;  // uniform per wave: later tiles are masked too
-                v4i kb[NV];
-                float ks_raw;
-                const uint32_t toff = buf * kKBuf + k * 32 * kRowBytes;
-                if constexpr (ELEM == 1) {
-                    lds_read_tile(ka[0] + toff, ka[1] + toff, ka[2] + toff, ka[3] + toff, ksa + buf * kSBuf + k * 128, kb,
-                                  ks_raw);
-                } else {
-                    lds_read_tile8(ka, toff, ksa + buf * kSBuf + k * 128, kb, ks_raw);
-                }
-                const float ks = ks_raw * (k < kPfTiles / 2 ? page_ok0 : page_ok1);
+                const float ks = pages_ok ? ks_raw : ks_raw * (k < kPfTiles / 2 ? page_ok0 : page_ok1);
                 // Units u = (row q = u / MT, head tile mt = u % MT), two dependent K-slice MFMAs
                 // each. Unit u+1's MFMAs are issued between the 32 VALU ops (ReLU, weight FMA) of
                 // unit u's epilogue so that the matrix core and the VALU work side by side.
                 constexpr int U = kPfRowsPerWave * MT;
                 float pj[kPfRowsPerWave][4];
-    #pragma unroll
+#pragma unroll
                 for (int q = 0; q < kPfRowsPerWave; ++q) pj[q][0] = pj[q][1] = pj[q][2] = pj[q][3] = 0.f;
                 v16f acc[2];
-                acc[0] = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-                for (int st = 0; st < STEPS; ++st) Mma<ELEM>::step(st, qa[0][0], kb, acc[0]);
-                __builtin_amdgcn_sched_barrier(0);
-    #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int q = u / MT, mt = u % MT;
-                    v16f& cur = acc[u & 1];
+#pragma unroll
+                for (int u = -1; u < U; ++u) {  // step -1: unit 0's MFMAs
                     v16f& nxt = acc[(u + 1) & 1];
                     if (u + 1 < U) {
                         nxt = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
+#pragma unroll
                         for (int st = 0; st < STEPS; ++st) Mma<ELEM>::step(st, qa[(u + 1) / MT][(u + 1) % MT], kb, nxt);
                     }
-    #pragma unroll
-                    for (int r4 = 0; r4 < 4; ++r4) {
-    #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const float relu = __int_as_float(max(__float_as_int(cur[r4 * 4 + j]), 0));
-                            pj[q][j] = fmaf(relu, wr[q][mt * 16 + r4 * 4 + j], pj[q][j]);
+                    if (u >= 0) {
+                        const int q = u / MT, mt = u % MT;
+                        const v16f& cur = acc[u & 1];
+#pragma unroll
+                        for (int r4 = 0; r4 < 4; ++r4) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const float relu = __int_as_float(max(__float_as_int(cur[r4 * 4 + j]), 0));
+                                pj[q][j] = fmaf(relu, wr[q][mt * 16 + r4 * 4 + j], pj[q][j]);
+                            }
                         }
                     }
-                    if (u + 1 < U) {
-                        // The next unit's STEPS MFMAs spread over this unit's 32 VALU ops (fp8:
-                        // 1 MFMA, 16 VALU, 1 MFMA, 16 VALU; bf16: 1 MFMA, 4 VALU, ...); nothing
-                        // crosses into the next unit.
-    #pragma unroll
+                    if (u >= 0 && u + 1 < U) {
+                        // The next unit's STEPS MFMAs spread over this unit's 32 VALU ops (1 MFMA, 16
+                        // VALU, 1 MFMA, 16 VALU); nothing crosses into the next unit.
+#pragma unroll
                         for (int st = 0; st < STEPS; ++st) {
                             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                             __builtin_amdgcn_sched_group_barrier(0x002, 32 / STEPS, 0);
                         }
+                    }
+                    if (u + 1 < U) __builtin_amdgcn_sched_barrier(0);
+                    if (u + 2 == U) {  // the tile's last MFMAs are issued
+                        load_tile(min(k + 1, kPfTiles - 1), kb, ks_raw);
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                // Two rows finish together: after the swap, lanes 0-31 hold row 0's total for
-                // token n and lanes 32-63 row 1's (each the sum of the two lane halves' heads).
-                // One row: both halves hold its total.
+                // The two rows finish together: after the swap [row 0 lanes 0-31, row 1 lanes 0-31] +
+                // [row 0 lanes 32-63, row 1 lanes 32-63], i.e. lanes 0-31 hold row 0's total for token n
+                // and lanes 32-63 row 1's.
                 const float part0 = (pj[0][0] + pj[0][1]) + (pj[0][2] + pj[0][3]);
-                float mine = part0, other = part0;
-                if constexpr (kPfRowsPerWave == 2) {
-                    const float part1 = (pj[1][0] + pj[1][1]) + (pj[1][2] + pj[1][3]);
-                    mine = g == 0 ? part0 : part1;
-                    other = g == 0 ? part1 : part0;
-                }
-                const auto swapped =
-                    __builtin_amdgcn_permlane32_swap(__float_as_int(other), __float_as_int(other), false, false);
-                const float total = mine + __int_as_float(g == 0 ? swapped[1] : swapped[0]);
-                const uint32_t key = sortable_key(bf16_bits_half_away(total * ks));
-                if (kPfRowsPerWave == 2 || g == 0) lds_write_b16(keya + k * 64, key);
-                if (t0 + n < vis_mine) {
-                    // Bins b and b ^ 128 share a word: the populated bins of a row are adjacent
-                    // and would otherwise serialise on one word's atomics.
-                    const uint32_t bin = key >> 8;
-                    lds_add_u32(hista + (bin & 127) * 4, 1u << (16 * (bin >> 7)));
-                }
+                const float part1 = (pj[1][0] + pj[1][1]) + (pj[1][2] + pj[1][3]);
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(part0), __float_as_int(part1), false, false);
+                const float total = __int_as_float(sw[0]) + __int_as_float(sw[1]);
+                const uint32_t key = score_key(total * ks);
+                *(LdsU16)(keya + k * 64) = static_cast<uint16_t>(key);
+                if (k * 32 < left) pf_count(hista, key);
             }
         }
         // Flush the chunk's keys of the wave's rows (8-byte stores, inside the row stride).
@@ -419,7 +423,7 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
         for (int q = 0; q < kPfRowsPerWave; ++q) {
             if (cstart >= vis[q]) continue;  // uniform
             const int o = min(lane * 4, kPfChunk - 4);
-            const v2i v = lds_read_b64(lds_addr(&s_keys[wave][q][o]));
+            const v2i v = *reinterpret_cast<const v2i*>(&s_keys[wave][q][o]);
             if (lane * 4 < kPfChunk && cstart + o + 4 <= p.key_stride) {
                 *reinterpret_cast<v2i*>(p.score_keys + static_cast<size_t>(rowi[q]) * p.key_stride + cstart + o) = v;
             }

@@ -163,7 +163,7 @@ KVIP_DEVICE uint32_t rg_key(const v4i (&qa)[MT][4], const float (&wr)[MT * 16], 
     float part = (pj[0] + pj[1]) + (pj[2] + pj[3]);
     const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_int(part), __float_as_int(part), false, false);
     part += __int_as_float(g == 0 ? swapped[1] : swapped[0]);
-    return sortable_key(bf16_bits_half_away(part * ks));
+    return score_key(part * ks);
 }
 
 template <int HEADS, bool W_BF16>
@@ -431,7 +431,7 @@ KVIP_DEVICE uint32_t rg_key2(const v4i (&qa)[MT][4], const float (&wr)[MT * 16],
     // [A lanes 0-31, B lanes 0-31] and [A lanes 32-63, B lanes 32-63].
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_int(part_a), __float_as_int(part_b), false, false);
     const float part = __int_as_float(sw[0]) + __int_as_float(sw[1]);
-    return sortable_key(bf16_bits_half_away(part * ks));
+    return score_key(part * ks);
 }
 
 // The eight 16-byte K fragment pieces of token rows n (A) and 32 + n (B, 4 KiB further) and

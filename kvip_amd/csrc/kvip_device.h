@@ -22,19 +22,17 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 KVIP_DEVICE int lane_id() { return __lane_id(); }
 
-// fp32 -> bf16 bits, rounding half away from zero on the magnitude (the Ascend
-// CAST_ROUND mode the reference scores use: tests/operators/lifetch/support/
-// workloads.py:233-235, op_kernel/indexer/indexer_score.h:105-140).
-KVIP_DEVICE uint32_t bf16_bits_half_away(float x) {
-    return (__float_as_uint(x) + 0x8000u) >> 16;
-}
-
-// bf16 bits -> order-preserving uint16 key (op_kernel/indexer/score_common.h:66-97):
-// the canonical NaN 0x7FC0 becomes 0xFFFF first; negative values are inverted,
-// non-negative values get the sign bit flipped.
-KVIP_DEVICE uint32_t sortable_key(uint32_t bits) {
-    bits = (bits == 0x7FC0u) ? 0xFFFFu : bits;
-    return (bits & 0x8000u) ? (~bits & 0xFFFFu) : (bits ^ 0x8000u);
+// fp32 score -> order-preserving 16-bit key: bf16 bits rounded half away from zero on the
+// magnitude (the Ascend CAST_ROUND mode the reference scores use: tests/operators/lifetch/
+// support/workloads.py:233-235, op_kernel/indexer/indexer_score.h:105-140), then negative values
+// inverted and non-negative ones with the sign bit flipped, the canonical NaN 0x7FC0 (flipped:
+// 0xFFC0) counting as 0xFFFF, whose key is 0 (op_kernel/indexer/score_common.h:66-97). Sign and
+// flip are taken on the rounded 32-bit pattern, which saves a shift and a select per key.
+KVIP_DEVICE uint32_t score_key(float x) {
+    const uint32_t v = __float_as_uint(x) + 0x8000u;
+    const uint32_t flip = static_cast<uint32_t>(static_cast<int32_t>(v) >> 31) | 0x80000000u;
+    const uint32_t key = (v ^ flip) >> 16;
+    return key == 0xFFC0u ? 0u : key;
 }
 
 KVIP_DEVICE float bf16_to_float(uint16_t bits) { return __uint_as_float(static_cast<uint32_t>(bits) << 16); }

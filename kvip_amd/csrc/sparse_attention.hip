@@ -106,7 +106,6 @@ __host__ __device__ inline int sa_splits(int rows, int heads) {
     return best;
 }
 
-typedef __attribute__((address_space(3))) const v4i* LdsV4i;
 typedef __attribute__((address_space(3))) const f32x4* LdsF32x4;
 typedef __attribute__((address_space(3))) i32x2* LdsI32x2;
 
@@ -130,18 +129,6 @@ KVIP_DEVICE bf16x8 fp8x8_to_bf16(int lo, int hi) {
         __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, false)),
         __builtin_bit_cast(int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.0f, true))};
     return __builtin_bit_cast(bf16x8, r);
-}
-
-// Direct-to-LDS loads as inline asm: 16 (4) bytes per lane from src to lds + lane * 16 (4),
-// lds wave-uniform. LLVM waits for every pending load of the builtin form before each LDS read;
-// the asm form is waited for explicitly once per tile, and the LDS reads stay ordinary code. The
-// loads have no output registers, so nothing can be reused while they are in flight; no other
-// instruction of the kernel uses m0.
-KVIP_DEVICE void dma16(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory");
-}
-KVIP_DEVICE void dma4(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory");
 }
 
 // Max / sum over lanes l, l ^ 16, l ^ 32, l ^ 48.
