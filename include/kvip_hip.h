@@ -601,7 +601,7 @@ uint32_t kvip_hip_topk(const KvipTopkArgs* args, void* stream);
 uint32_t kvip_hip_fetch_gather(const KvipFetchArgs* args, void* stream);
 uint32_t kvip_hip_indexer_prefill(const KvipPrefillArgs* args, void* stream);
 /* kvip_hip_indexer_prefill on a grid of at most `workgroups` workgroups (0: one per work unit
- * of 8 query rows x 4096 key positions, as kvip_hip_indexer_prefill) that stride over the
+ * of 8 query rows x up to 4096 key positions, as kvip_hip_indexer_prefill) that stride over the
  * units; same results. No reference counterpart: a launch shape for callers that run the
  * prefill beside other kernels (a mixed decode + prefill round), where a grid of twice the
  * CU count leaves the CUs that finish their units to the other kernels. */

@@ -3,7 +3,7 @@
 // or bf16 Q/K.
 //
 // Work unit = (query block, context segment): 8 consecutive query rows of one sequence
-// against 4096 key positions (one unit per workgroup, or a bounded grid whose workgroups
+// against up to 4096 key positions (one unit per workgroup, or a bounded grid whose workgroups
 // stride over the units, kvip_hip_indexer_prefill_grid). fp8: 4 waves own 2 query rows
 // each; bf16 (Q fragments twice as large): 8 waves own one row each. A wave keeps its rows'
 // Q fragments and per-lane head weights (w'_h = w_h * qscale_h for the 32 heads a lane
@@ -57,7 +57,8 @@ struct PfShape {
     static constexpr int kRows = kPfBlockRows / kWaves;
     static constexpr int kThreads = kWaves * 64;
 };
-constexpr int kPfSegment = 4096;                            // key positions per workgroup
+constexpr int kPfChunk = 256;                               // key positions staged at a time
+constexpr int kPfSegment = 4096;                            // most key positions per work item
 constexpr int kPfPages = kPfSegment / kBlockTokens;         // 32
 constexpr int kPfMaxSeq = KVIP_PREFILL_MAX_SEQUENCES;
 // LDS piece swizzle of a staged K row of 8 (fp8) or 16 (bf16) 16-byte pieces: piece j of
@@ -87,19 +88,18 @@ KVIP_DEVICE void pf_count(uint32_t hist, uint32_t key) {
 }
 
 template <int ELEM, int HEADS, bool W_BF16>
-__global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_prefill_kernel(const KvipPrefillArgs p) {
+__global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_prefill_kernel(const KvipPrefillArgs p, const int segment) {
     constexpr int kPfWaves = PfShape<ELEM>::kWaves;
     constexpr int kPfRowsPerWave = PfShape<ELEM>::kRows;
     constexpr int kPfThreads = PfShape<ELEM>::kThreads;
-    constexpr int kPfChunkBytes = 256 * kIndexDim * ELEM;  // 256 tokens per LDS chunk
+    constexpr int kPfChunkBytes = kPfChunk * kIndexDim * ELEM;
     constexpr int MT = HEADS / 32;
     constexpr int NV = Mma<ELEM>::NV;              // 16-byte pieces of a half row per lane
     constexpr int STEPS = Mma<ELEM>::STEPS;        // MFMAs per 128-dim contraction
     constexpr int kRowBytes = kIndexDim * ELEM;
     constexpr int kPieces = kRowBytes / 16;        // 16-byte pieces per K row
-    constexpr int kPfChunk = kPfChunkBytes / kRowBytes;  // tokens per LDS chunk (256 or 128)
     constexpr int kPfTiles = kPfChunk / 32;
-    constexpr int kChunkPages = kPfChunk / kBlockTokens;  // pages per chunk (2 or 1)
+    constexpr int kChunkPages = kPfChunk / kBlockTokens;  // pages per chunk (2)
     constexpr int kRowsPerLoad = 64 / kPieces;     // K rows one 64-lane 16-byte load fills
     static_assert(kPfRowsPerWave == 1 || kPfRowsPerWave == 2, "the finish maps row q to lane half q");
     constexpr int kStageLoads = (kPfChunk / kPfWaves) / kRowsPerLoad;  // staging loads per wave and chunk
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
     // of queueing more items behind the other kernels).
     const int nb_items = p.rows / kPfBlockRows + p.sequences;
     const int64_t n_items =
-        static_cast<int64_t>(nb_items) * ((p.max_blocks * kBlockTokens + kPfSegment - 1) / kPfSegment);
+        static_cast<int64_t>(nb_items) * ((p.max_blocks * kBlockTokens + segment - 1) / segment);
     uint32_t err = 0;
     for (int64_t item = blockIdx.x; item < n_items; item += gridDim.x) {
     const int block = static_cast<int>(item) % nb_items;  // n_items <= 2^31 - 1 (validated)
@@ -173,8 +173,8 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
     }
     const int last = min(j0 + kPfBlockRows, q_len) - 1;
     const int vis_max = min(max(k_len - q_len + last + 1, 0), k_len);
-    const int seg0 = segi * kPfSegment;
-    const int seg_end = min(seg0 + kPfSegment, vis_max);
+    const int seg0 = segi * segment;
+    const int seg_end = min(seg0 + segment, vis_max);
     if (seg0 >= seg_end) continue;  // uniform: nothing visible in this segment
     const int nchunks = (seg_end - seg0 + kPfChunk - 1) / kPfChunk;
 
@@ -451,21 +451,54 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
 }
 
 // Work items: (query blocks bound) x (segments of the bound context).
-int64_t prefill_items(const KvipPrefillArgs& a) {
+int64_t prefill_items(const KvipPrefillArgs& a, int segment) {
     const int64_t blocks = a.rows / kPfBlockRows + a.sequences;  // bound on the per-sequence blocks
-    return blocks * ((static_cast<int64_t>(a.max_blocks) * kBlockTokens + kPfSegment - 1) / kPfSegment);
+    return blocks * ((static_cast<int64_t>(a.max_blocks) * kBlockTokens + segment - 1) / segment);
+}
+
+// Key positions per work item. With few items a long segment leaves CUs idle (one chunk of 256
+// keys takes about 5 us, 16 of them 80 us) or ends in a last round that few of them share; a short
+// one pays an item's Q fragments, staging latency and histogram flush more often. The launch is
+// priced as (all items, or one per CU, + a tail from uneven items) x (lead + chunks) in chunk times
+// and the cheapest segment taken. Lead and tail are fitted to every segment measured at 16
+// shapes of 16 to 8192 rows against 1024 to 65536 keys: lead 0.5 and tail 1 for fp8, 1.25 and
+// 0.25 for bf16 (twice the Q, one workgroup per CU); the choice is within 1% (fp8) and 3% (bf16) of
+// the best segment on average, 19% at worst. Against 4096 keys throughout, us fp8 / bf16: 16 rows x
+// 4096 keys 80.5 -> 11.7 / 89.1 -> 13.9, 64 x 16384 81.2 -> 24.1 / 92.4 -> 34.7, 512 x 8192 81.4 ->
+// 43.2 / 98.6 -> 75.9, six sequences of 33-900 rows 121.3 -> 103.5 / 199.9 -> 187.0, 4096 x 16384
+// 478 -> 459 / 840 -> 840. Long segments stay where items are many: 2048 x 65536 takes 974 us with
+// 4096 keys and 1447 with 256.
+int prefill_segment(const KvipPrefillArgs& a, int workgroups) {
+    constexpr int kCus = 256;
+    const int64_t cus = workgroups > 0 ? std::min(workgroups, kCus) : kCus;
+    const bool fp8 = a.qk_dtype == KVIP_DTYPE_FP8_E4M3;
+    const int64_t lead = fp8 ? 2 : 5, tail = fp8 ? 4 : 1;  // quarters of a chunk, of an item per CU
+    const int64_t context_chunks = (static_cast<int64_t>(a.max_blocks) * kBlockTokens + kPfChunk - 1) / kPfChunk;
+    // Likely blocks (prefill_items has the bound): a further sequence ends in half a block on average.
+    const int64_t blocks = (a.rows + kPfBlockRows / 2 * (a.sequences - 1) + kPfBlockRows - 1) / kPfBlockRows;
+    int best = kPfSegment;
+    int64_t best_cost = INT64_MAX;
+    for (int segment = kPfSegment; segment >= kPfChunk; segment /= 2) {
+        if (prefill_items(a, segment) > INT32_MAX) break;  // the kernel's item index
+        const int64_t items = blocks * ((static_cast<int64_t>(a.max_blocks) * kBlockTokens + segment - 1) / segment);
+        const int64_t item = lead + 4 * std::min<int64_t>(segment / kPfChunk, context_chunks);
+        const int64_t cost = 4 * std::max(items * lead + blocks * 4 * context_chunks, cus * item) + tail * cus * item;
+        if (cost < best_cost) best = segment, best_cost = cost;
+    }
+    return best;
 }
 
 template <int ELEM, int HEADS>
 hipError_t launch_heads(const KvipPrefillArgs& a, int workgroups, hipStream_t stream) {
-    const int64_t items = prefill_items(a);
+    const int segment = prefill_segment(a, workgroups);
+    const int64_t items = prefill_items(a, segment);
     const dim3 grid(static_cast<unsigned>(workgroups > 0 ? std::min<int64_t>(items, workgroups) : items));
     if (a.weight_dtype == KVIP_DTYPE_BF16) {
         hipLaunchKernelGGL((indexer_prefill_kernel<ELEM, HEADS, true>), grid, dim3(PfShape<ELEM>::kThreads), 0, stream,
-                           a);
+                           a, segment);
     } else {
         hipLaunchKernelGGL((indexer_prefill_kernel<ELEM, HEADS, false>), grid, dim3(PfShape<ELEM>::kThreads), 0, stream,
-                           a);
+                           a, segment);
     }
     return hipGetLastError();
 }
@@ -492,7 +525,7 @@ uint32_t validate_prefill(const KvipPrefillArgs* a) {
         (a->key_scale == nullptr || (a->scale_block_stride >= kBlockTokens && a->scale_block_stride % 4 == 0 &&
                                      (reinterpret_cast<uintptr_t>(a->key_scale) & 15u) == 0)) &&
         aligned16(a->query) && aligned16(a->keys) && aligned16(a->score_keys) &&
-        prefill_items(*a) <= 0x7FFFFFFF;
+        prefill_items(*a, kPfSegment) <= 0x7FFFFFFF;
     return ok ? KVIP_OK : KVIP_ERR_INVALID;
 }
 

@@ -48,7 +48,7 @@ class PrefillIndexer:
         self.topk = torch.full((max_rows, TOPK), -1, dtype=torch.int32, device=dev)
         self.status = torch.zeros(1, dtype=torch.int32, device=dev)
         self.library = abi.load_library()
-        # Scoring grid: 0 = one workgroup per work unit (8 query rows x 4096 key positions);
+        # Scoring grid: 0 = one workgroup per work unit (8 query rows x up to 4096 keys);
         # n > 0 = at most n workgroups striding over the units (kvip_hip_indexer_prefill_grid),
         # for rounds that run other kernels beside the prefill.
         self.workgroups = 0

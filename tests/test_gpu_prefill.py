@@ -165,6 +165,39 @@ def test_prefill_bounded_grid_equals_full_grid(torch_gpu, qk, workgroups):
     assert h0.sum() == v0.sum()
 
 
+@pytest.mark.parametrize("qk", ["fp8", "bf16"])
+@pytest.mark.parametrize("rows,k_len", [(2050, 9001), (600, 9100), (130, 19999), (1024, 2049), (16, 4097)])
+def test_prefill_rows_do_not_depend_on_the_segment(torch_gpu, qk, rows, k_len):
+    """The launch picks 256 to 4096 keys per work item by rows and context: 1024, 512, 512, 512 and
+    256 here for fp8, 4096, 2048, 1024, 1024 and 256 for bf16. A sequence's last 9 rows scored alone (256 keys per item, few items) see the same keys as the
+    same rows of the whole sequence, so keys, histograms and TopK are the same, bit for bit."""
+    torch = torch_gpu
+    say(f"case prefill segment {qk} rows={rows} k_len={k_len}")
+    c = make_case(torch, q_lens=[rows], k_lens=[k_len], heads=64, wdt=torch.float32, qscale=True, kscale=True,
+                  seed=41, qk=qk)
+
+    def score(first):
+        n = rows - first
+        idx = kvip_amd.PrefillIndexer(torch, max_rows=n, max_context=c["max_ctx"], max_sequences=1, device="cuda")
+        idx.bind(c["query"][first:], c["weights"][first:], c["query_scale"][first:], c["keys"], c["key_scale"],
+                 torch.tensor([0, n], dtype=torch.int32, device="cuda"), c["kl"], c["table"])
+        idx.score()
+        torch.cuda.synchronize()
+        keys, vis, hist = idx.score_keys.clone(), idx.row_valid.clone(), idx.histogram.clone()
+        top = idx.select().clone()
+        assert int(idx.status.item()) == 0
+        return keys, vis, hist, top
+
+    whole, last = score(0), score(rows - 9)
+    assert torch.equal(whole[1], torch.arange(k_len - rows + 1, k_len + 1, device="cuda", dtype=torch.int32))
+    assert torch.equal(whole[2].sum(1, dtype=torch.int32), whole[1])
+    for q in range(9):
+        r, n = rows - 9 + q, k_len - 8 + q
+        assert torch.equal(whole[0][r, :n], last[0][q, :n])
+    for a, b in zip(whole[1:], last[1:]):
+        assert torch.equal(a[rows - 9:], b)
+
+
 def test_quant_lightning_indexer_wrapper(torch_gpu):
     """The native-call surface: TND rows, cumulative query lengths, [blocks,128,1,128] keys."""
     torch = torch_gpu
