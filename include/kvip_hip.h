@@ -609,7 +609,8 @@ uint32_t kvip_hip_indexer_prefill_grid(const KvipPrefillArgs* args, int32_t work
 uint32_t kvip_hip_lifetch_forward(const KvipLIFetchArgs* args, void* stream);
 /* The launch plan kvip_hip_lifetch_forward takes for these arguments (no launch, no device
  * access): KVIP_LIFETCH_PLAN_THREE (scoring, TopK, gather; rows of at most
- * KVIP_TOPK_REGS_MAX_KEYS keys use the register-resident TopK), or KVIP_ERR_INVALID when
+ * KVIP_TOPK_REGS_MAX_KEYS keys use the register-resident TopK; up to 16 query rows of at most
+ * 32768 keys with topk.segments given run TopK and gather as one launch), or KVIP_ERR_INVALID when
  * the forward would reject them. A host query with no counterpart in the reference, for
  * callers and tests that need to know which kernels a round runs. */
 #define KVIP_LIFETCH_PLAN_THREE 0u

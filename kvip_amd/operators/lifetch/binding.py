@@ -140,8 +140,9 @@ class LIFetchBinding:
         )
 
     def topk_args(self, use_histogram=True, split=True):
-        """TopK arguments; with the scoring histogram the select runs on 4096-key segments
-        (split=True) or one workgroup per row (split=False)."""
+        """TopK arguments; with the scoring histogram a row is selected in 2048-key
+        segments (8192-key ones above 65536 keys) by many workgroups (split=True), or by one
+        workgroup (split=False)."""
         p = abi.ptr
         return abi.TopkArgs(
             score_keys=p(self.score_keys), histogram=p(self.histogram) if use_histogram else 0,

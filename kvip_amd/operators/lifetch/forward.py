@@ -234,6 +234,6 @@ class LIFetchForward:
 
     def select_fetch(self):
         """TopK fused with the Fetch gather in one launch (kvip_hip_select_fetch; needs the
-        binding's segment work memory and rows of at most 32768 keys). Not part of the
-        default forward, whose separate gather launch measured faster."""
+        binding's segment work memory and rows of at most 32768 keys). The forward takes it by
+        itself for up to 16 query rows; with more rows its separate gather launch is faster."""
         abi.check(self.library.kvip_hip_select_fetch(self._topk, self._fetch, self._stream()), "TopK+Fetch")
