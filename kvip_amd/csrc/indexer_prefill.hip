@@ -463,14 +463,17 @@ int64_t prefill_items(const KvipPrefillArgs& a, int segment) {
 // and the cheapest segment taken. Lead and tail are fitted to every segment measured at 16
 // shapes of 16 to 8192 rows against 1024 to 65536 keys: lead 0.5 and tail 1 for fp8, 1.25 and
 // 0.25 for bf16 (twice the Q, one workgroup per CU); the choice is within 1% (fp8) and 3% (bf16) of
-// the best segment on average, 19% at worst. Against 4096 keys throughout, us fp8 / bf16: 16 rows x
-// 4096 keys 80.5 -> 11.7 / 89.1 -> 13.9, 64 x 16384 81.2 -> 24.1 / 92.4 -> 34.7, 512 x 8192 81.4 ->
-// 43.2 / 98.6 -> 75.9, six sequences of 33-900 rows 121.3 -> 103.5 / 199.9 -> 187.0, 4096 x 16384
-// 478 -> 459 / 840 -> 840. Long segments stay where items are many: 2048 x 65536 takes 974 us with
-// 4096 keys and 1447 with 256.
+// the best segment on average, 19% at worst. Against 4096 keys throughout, scoring alone, us fp8 /
+// bf16: 16 rows x 4096 keys 84.6 -> 11.7 / 100.6 -> 13.8, 64 x 16384 86.3 -> 24.0 / 102.8 -> 41.7, 512 x
+// 8192 88.0 -> 49.8 / 104.2 -> 66.8, six sequences of 33-900 rows 125 -> 106 / 199 -> 190, 4096 x 16384
+// 497 -> 466 / 886 -> 854. Long segments stay where items are many: 2048 x 65536 takes 974 us with
+// 4096 keys and 1447 with 256. A bounded grid keeps 4096 keys: its launch runs beside other kernels,
+// which take the CUs of the workgroups that run out of items, and items of equal size would hold all
+// of them to the end (a round of 32 decode requests beside chunks of 2048 x 8192 and 1536 x 1536:
+// 307-310 us with short segments, 276-279 with these).
 int prefill_segment(const KvipPrefillArgs& a, int workgroups) {
-    constexpr int kCus = 256;
-    const int64_t cus = workgroups > 0 ? std::min(workgroups, kCus) : kCus;
+    if (workgroups > 0) return kPfSegment;
+    constexpr int64_t cus = 256;
     const bool fp8 = a.qk_dtype == KVIP_DTYPE_FP8_E4M3;
     const int64_t lead = fp8 ? 2 : 5, tail = fp8 ? 4 : 1;  // quarters of a chunk, of an item per CU
     const int64_t context_chunks = (static_cast<int64_t>(a.max_blocks) * kBlockTokens + kPfChunk - 1) / kPfChunk;
