@@ -18,9 +18,10 @@
 //   - A tile stays as it is in the cache: direct-to-LDS loads put its 512 fp8 bytes per token into a
 //     two-slot ring, tile k + 4 landing while tile k is computed. No dequantised copy is made.
 //   - Logits: fp8 MFMA (16x16x128, one scale group per instruction) of the raw key bytes with the
-//     query as two fp8 terms, which hold bf16's eight significant bits, so no key byte is
+//     query as two fp8 terms, which hold bf16's eight significant bits over 2^14, so no key byte is
 //     converted; each scale group's dot products are summed on their own and added as
-//     fma(group, scale, s) in fp32. The rope features are bf16 MFMA.
+//     fma(group, scale, s) in fp32. A query whose features lie further apart (sa_wide) stays bf16 and
+//     the key bytes are converted (exactly) for bf16 MFMA. The rope features are bf16 MFMA.
 //   - Values: bf16 MFMA of the value bytes, converted as they are read (two features per
 //     v_cvt_scalef32_pk_bf16_fp8 with scale 1, exact), with the probabilities times the group's
 //     scale (fp32, then rounded to bf16). One rounding per product instead of one on either side.
@@ -39,11 +40,15 @@
 // (about 620 instructions per wave and tile). LDS (ring 128 KB, rope 16 KB, cache rows 8 KB,
 // scales 4 KB) allows one workgroup per CU. Measured, 64 rows, against the version that
 // dequantised tiles to bf16 in LDS and exchanged probabilities between waves: 16 heads of 16384
-// hot slots 37.6 -> 30.4 us per call, 128 heads of 2048 slots 98.8 -> 71.8; 32 heads 47.1 -> 34.4,
-// 64 heads 58.2 -> 45.4; one row of 16 heads 21.7 -> 13.0. Error against 64 bits on N(0, 1) rows:
-// 1.1e-3 (1.9e-3 with both sides rounded).
+// hot slots 37.4 -> 30.7 us per call, 128 heads of 2048 slots 98.7 -> 72.3; 32 heads 47.1 -> 34.4,
+// 64 heads 58.2 -> 45.4; one row of 16 heads 21.8 -> 12.8. Error against 64 bits on N(0, 1) rows:
+// 1.1e-3 (1.9e-3 with both sides rounded). Looking the query over for far smaller features takes 0.3 us
+// of a call; one that has them takes 14.9 us for one row, 30.5 for 64 rows of 16 heads and
+// 78.6 of 128 (that version: 21.8, 35.5, 96.9; two terms alone: 12.5, 27.5, 68.1).
 // A variant with groups of 32 heads per wave (32x32x16 MFMA, 256 accumulators) spilled (356 us at 128
 // heads); scratch reloads wait for every load in flight, so the tile loop must not spill.
+#include <type_traits>
+
 #include "lds_async.h"
 
 namespace kvip {
@@ -54,14 +59,17 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef int i32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
 
 constexpr int kSaHeads = 16;                // heads per wave (MFMA N)
 constexpr int kSaStreams = 4;               // token streams per workgroup
 constexpr int kSaTile = 32;                 // tokens per tile (value MFMA K)
 constexpr int kKeyDim = 576;                // 512 nope + 64 rope
 constexpr int kValueDim = 512;
-constexpr int kScaleGroups = 4;             // 128 nope features share a scale
+constexpr int kScaleGroups = 4;
+constexpr int kGroupDim = kValueDim / kScaleGroups;  // nope features that share a scale
 constexpr int kMaxSplits = 16;
+constexpr int kWideMark = 256;              // in place of a query exponent: the query stays bf16
 constexpr int kPartial = kValueDim + 2;     // floats per (row, head, split): output, max, sum
 constexpr float kLog2e = 1.44269504088896341f;
 constexpr float kSaMargin = 8.0f * kLog2e;  // lazy rescale: 8 in natural-log units
@@ -150,6 +158,15 @@ KVIP_DEVICE float rows4_sum(float x) {
 // tokens) and a value read (two 16-lane blocks of a transpose load: one piece of the 8 tokens
 // 4 kg .. + 3 and 16 + 4 kg .. + 3 for kg and kg + 1) touch every bank once.
 KVIP_DEVICE constexpr int sa_swz(int t) { return (t & 7) | ((((t >> 3) ^ (t >> 4)) & 1) << 3); }
+
+// Whether a query must stay bf16, by one head's scale group: `held` of its features lie within 2^13 of
+// the largest one's power of two (2^14 where that is even), where the two fp8 terms are exact, and
+// `tiny` nonzero ones lie below, where the terms are off by up to 2^-22 of the largest. With 32 held
+// features beside each tiny one (so at most three of the 128 are) that error is lost. With fewer, a
+// key that is zero at the large features would show it. An infinity or NaN (`top`, the largest biased
+// exponent, is 255) has no terms. N(0, 1) queries have one tiny feature in about 60 groups and hardly
+// ever four in one.
+KVIP_DEVICE bool sa_wide(int top, int held, int tiny) { return top == 255 || 32 * tiny > held; }
 
 // 16 tokens x 16 heads over 128 features: fp8 keys (scale 1) by fp8 query terms with block scale
 // byte g of `scales`.
@@ -331,24 +348,38 @@ __global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kerne
     load_rope();
     report(p.status, err);
 
-    // The query as two fp8 e4m3 terms, q = (hi + lo) * 2^e with one e per head and 128 features (the
-    // block scale of the MFMA): hi takes the upper four of bf16's eight significant bits, lo the rest. That is exact
-    // for features within 2^9 of their group's largest and off by at most 2^-17 of the largest for
-    // smaller ones; a group with an infinity or NaN gets the NaN scale.
-    // Wave st converts group st; the terms go through LDS (the ring's second slots, free until the
-    // first tile has landed) to the waves of the other streams.
+    // The query as two fp8 e4m3 terms, q = (hi + lo 2^-5) 2^e with one e per head and 128 features (the
+    // block scales of the MFMA): hi takes the upper four of bf16's eight significant bits, lo the rest
+    // (at most 2^3 where the largest feature is below 2^8, so 2^8 after its scale). That is exact
+    // down to 2^-14 of the largest feature; with more features below it than sa_wide allows, the
+    // whole workgroup's query stays bf16. Wave st converts group st; the terms go through LDS (the ring's second
+    // slots, free until the first tile has landed) to the waves of the other streams.
     v4i* s_qf = reinterpret_cast<v4i*>(s_mem + kNopeSlot) + gi * 256;  // + stream * 2 slots: its group's terms
     int* s_qe = reinterpret_cast<int*>(s_mem + kLdsQuery);             // [group of heads][head][scale group]
     {
-        uint32_t top = 0;
+        // Two features to a register, sign bits set: their largest by magnitude.
+        auto features = [&](int x) { return static_cast<uint32_t>(qraw[x >> 2][x & 3]) | 0x80008000u; };
+        u16x2 largest = __builtin_bit_cast(u16x2, features(0));
 #pragma unroll
-        for (int x = 0; x < 16; ++x) {
-            const uint32_t v = static_cast<uint32_t>(qraw[x >> 2][x & 3]);
-            top = max(top, max(v & 0x7FFFu, (v >> 16) & 0x7FFFu));
-        }
-        top = static_cast<uint32_t>(rows4_max(static_cast<float>(top >> 7)));  // over the group's four lanes
-        const int e = max(static_cast<int>(top), 8);        // biased exponent of the largest
+        for (int x = 1; x < 16; ++x) largest = __builtin_elementwise_max(largest, __builtin_bit_cast(u16x2, features(x)));
+        const int top = static_cast<int>(rows4_max(static_cast<float>((max(largest[0], largest[1]) & 0x7FFF) >> 7)));
+        const int e = max(top, 13);                         // biased exponent of the largest
         const float mul = __int_as_float((261 - e) << 23);  // 2^(134 - e): the largest below 2^8
+        // How many of the group's features are at least 2^(2 k) (pairs of exponents, so that four features'
+        // high bytes share a register): with the sign bits set, a subtraction leaves the bit where the byte
+        // is not below what is taken away, and borrows nothing across.
+        auto at_least = [&](int k) {
+            int count = 0;
+#pragma unroll
+            for (int x = 0; x < 16; x += 2) {
+                const uint32_t high = __builtin_amdgcn_perm(features(x), features(x + 1), 0x07050301u);
+                count += __popc((high - static_cast<uint32_t>(k) * 0x01010101u) & 0x80808080u);
+            }
+            return static_cast<int>(rows4_sum(static_cast<float>(count)));
+        };
+        const int held = at_least((max(e - 14, 1) + 1) >> 1);
+        bool wide = sa_wide(top, held, kGroupDim - held);    // zeros taken for tiny ones
+        if (__ballot(wide) != 0ull) wide = sa_wide(top, held, at_least(1) - held);
         v4i* dst = s_qf + st * (2 * kNopeSlot / 16) + lane;
 #pragma unroll
         for (int half = 0; half < 2; ++half) {  // features of the lane's first, second piece
@@ -362,8 +393,8 @@ __global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kerne
                     const float a = __uint_as_float(v << 16) * mul, c = __uint_as_float(v & 0xFFFF0000u) * mul;
                     h = y ? __builtin_amdgcn_cvt_pk_fp8_f32(a, c, h, true) : __builtin_amdgcn_cvt_pk_fp8_f32(a, c, h, false);
                     const f32x2 back = y ? __builtin_amdgcn_cvt_pk_f32_fp8(h, true) : __builtin_amdgcn_cvt_pk_f32_fp8(h, false);
-                    l = y ? __builtin_amdgcn_cvt_pk_fp8_f32(a - back[0], c - back[1], l, true)
-                          : __builtin_amdgcn_cvt_pk_fp8_f32(a - back[0], c - back[1], l, false);
+                    const float ra = (a - back[0]) * 32.0f, rc = (c - back[1]) * 32.0f;
+                    l = y ? __builtin_amdgcn_cvt_pk_fp8_f32(ra, rc, l, true) : __builtin_amdgcn_cvt_pk_fp8_f32(ra, rc, l, false);
                 }
                 hi[x] = h;
                 lo[x] = l;
@@ -371,155 +402,200 @@ __global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kerne
             dst[half * 64] = hi;
             dst[(2 + half) * 64] = lo;
         }
-        if (kg == 0) s_qe[(gi * kSaHeads + n) * kScaleGroups + st] = e == 255 ? 255 : e - 7;
+        if (kg == 0) s_qe[(gi * kSaHeads + n) * kScaleGroups + st] = wide ? kWideMark : e - 7;
     }
     v4i* s_rope = reinterpret_cast<v4i*>(s_mem + kLdsQuery + 2 * kSaHeads * kScaleGroups * 4) + gi * 64;
     if (st == 0) s_qf[512 + lane] = qrope;  // past the terms of both head groups
     if (st == 1) s_rope[lane] = qrope;
     lds_sync();
     v8i qh[kScaleGroups], ql[kScaleGroups];
-    int qscale = 0;  // byte g: E8M0 scale of group g
+    int qscale = 0;  // byte g: E8M0 scale of group g's hi terms (lo: 5 less)
+    const v4i* s_qe4 = reinterpret_cast<const v4i*>(s_qe);
+    const v4i qe = s_qe4[gi * kSaHeads + n], qe_other = s_qe4[(G - 1 - gi) * kSaHeads + n];
+    bool wide = false;
 #pragma unroll
     for (int g = 0; g < kScaleGroups; ++g) {
         const v4i* src = s_qf + g * (2 * kNopeSlot / 16) + lane;
         const v4i a = src[0], c = src[64], d = src[128], f = src[192];
         qh[g] = v8i{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
         ql[g] = v8i{d[0], d[1], d[2], d[3], f[0], f[1], f[2], f[3]};
-        qscale |= s_qe[(gi * kSaHeads + n) * kScaleGroups + g] << (8 * g);
+        wide |= qe[g] == kWideMark || qe_other[g] == kWideMark;
+        qscale |= (qe[g] & 255) << (8 * g);
+    }
+    wide = __ballot(wide) != 0ull;  // the same in every wave: the copies of the tile loop hold barriers
+    const int qscale_lo = qscale - 0x05050505;  // every byte is at least 6 (unless wide)
+    if (wide) {  // the bf16 features of each group: the lane's first piece in qh, its second in ql
+        const uint16_t* q = p.query + (static_cast<size_t>(r) * p.heads + min(h0 + n, p.heads - 1)) * kKeyDim + kg * 16;
+#pragma unroll
+        for (int g = 0; g < kScaleGroups; ++g) {
+            const v4i* src = reinterpret_cast<const v4i*>(q + g * 128);
+            const v4i a = src[0], c = src[1], d = src[8], f = src[9];
+            qh[g] = v8i{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
+            ql[g] = v8i{d[0], d[1], d[2], d[3], f[0], f[1], f[2], f[3]};
+        }
+        // Waited for here: the tile loop would wait for them each time round, and so for its own loads.
+#pragma unroll
+        for (int g = 0; g < kScaleGroups; ++g) asm volatile("" : "+v"(qh[g]), "+v"(ql[g]));
     }
     const bf16x8 q_rope = __builtin_bit_cast(bf16x8, s_qf[512 + lane]);
     lds_sync();  // the ring's second slots are free
-    int slot = 0;
-    for (int k = st; k < tiles; k += kSaStreams, slot ^= 1) {
-        const bool more = k + kSaStreams < tiles;
-        settle(true);  // the tile has landed; the other slot is free
-        uint32_t next = 0;
-        if (more) {
-            next = describe(k + kSaStreams);
-            load_nope(slot ^ 1, next);
-        }
-        // LDS addresses of this lane's reads, derived anew for each tile (held over the loop they
-        // would cost registers that the accumulators need). Keys: piece 4 j + kg of token 16 u + n; the
-        // XOR with 64 j moves between pieces. Values: block kg of a transpose load covers 16 features
-        // (one piece) of the 8 tokens that lane group kg holds probabilities of: 4 kg + 0 .. 3 and
-        // 16 + 4 kg + 0 .. 3.
-        const int ln = fresh(lane), tn = ln & 15, tk = ln >> 4;
-        const uint32_t ro = rope_lds + tn * 128 + ((tk ^ ((tn >> 1) & 7)) << 4);
-        const uint32_t ko = ring_lds + slot * kNopeSlot + tn * kValueDim + ((tk ^ sa_swz(tn)) << 4);
-        const int vt = 4 * tk + ((tn >> 1) & 3) + 16 * (tn >> 3);
-        const uint32_t vo = ring_lds + slot * kNopeSlot + vt * kValueDim + (sa_swz(vt) << 4) + 8 * (ln & 1);
-        const uint32_t sl = scales_lds + slot * kScaleSlot + 16 * tk;  // scales of tokens 4 kg .. + 3
+    // The tiles of this wave's stream, in two copies: a branch within the loop spilled 76 registers.
+    auto stream = [&](auto wide_query) {
+        constexpr bool kWide = decltype(wide_query)::value;
+        int slot = 0;
+        for (int k = st; k < tiles; k += kSaStreams, slot ^= 1) {
+            const bool more = k + kSaStreams < tiles;
+            settle(true);  // the tile has landed; the other slot is free
+            uint32_t next = 0;
+            if (more) {
+                next = describe(k + kSaStreams);
+                load_nope(slot ^ 1, next);
+            }
+            // LDS addresses of this lane's reads, derived anew for each tile (held over the loop they
+            // would cost registers that the accumulators need). Keys: piece 4 j + kg of token 16 u + n; the
+            // XOR with 64 j moves between pieces. Values: block kg of a transpose load covers 16 features
+            // (one piece) of the 8 tokens that lane group kg holds probabilities of: 4 kg + 0 .. 3 and
+            // 16 + 4 kg + 0 .. 3.
+            const int ln = fresh(lane), tn = ln & 15, tk = ln >> 4;
+            const uint32_t ro = rope_lds + tn * 128 + ((tk ^ ((tn >> 1) & 7)) << 4);
+            const uint32_t ko = ring_lds + slot * kNopeSlot + tn * kValueDim + ((tk ^ sa_swz(tn)) << 4);
+            const int vt = 4 * tk + ((tn >> 1) & 3) + 16 * (tn >> 3);
+            const uint32_t vo = ring_lds + slot * kNopeSlot + vt * kValueDim + (sa_swz(vt) << 4) + 8 * (ln & 1);
+            const uint32_t sl = scales_lds + slot * kScaleSlot + 16 * tk;  // scales of tokens 4 kg .. + 3
 
-        // Logits [tokens, heads], lane: tokens 16 u + 4 kg + i of head n. Rope first, whose buffer
-        // then takes the next tile's rope.
-        f32x4 sv[2];
-        {
-            const v4i q1 = *(LdsV4i)lds_addr(s_rope + ln);
+            // Logits [tokens, heads], lane: tokens 16 u + 4 kg + i of head n. Rope first, whose buffer
+            // then takes the next tile's rope.
+            f32x4 sv[2];
+            {
+                const v4i q1 = *(LdsV4i)lds_addr(s_rope + ln);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const v4i k0 = *(LdsV4i)(ro + u * 16 * 128), k1 = *(LdsV4i)((ro ^ 64) + u * 16 * 128);
-                sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k0), q_rope,
-                                                                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k1),
-                                                                __builtin_bit_cast(bf16x8, q1), sv[u], 0, 0, 0);
+                for (int u = 0; u < 2; ++u) {
+                    const v4i k0 = *(LdsV4i)(ro + u * 16 * 128), k1 = *(LdsV4i)((ro ^ 64) + u * 16 * 128);
+                    sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k0), q_rope,
+                                                                    f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    sv[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k1),
+                                                                    __builtin_bit_cast(bf16x8, q1), sv[u], 0, 0, 0);
+                }
             }
-        }
-        settle(false);
-        if (more) load_rope();
-        if (live) {
-            // One scale group of 16 tokens per step (i: token half i / 4, group i % 4), its key bytes read
-            // one step ahead; the raw fp8 bytes are the A operand.
-            auto key = [&](int i) {
-                const uint32_t at = ko ^ ((i & 3) * 128) ^ (sa_swz(16 * (i >> 2)) * 16);
-                const v4i x = *(LdsV4i)(at + (i >> 2) * 16 * kValueDim);
-                const v4i y = *(LdsV4i)((at ^ 64) + (i >> 2) * 16 * kValueDim);
-                return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-            };
-            v8i kv[2] = {key(0), v8i{}};
+            settle(false);
+            if (more) load_rope();
+            if (live) {
+                // One scale group of 16 tokens per step (i: token half i / 4, group i % 4), its key bytes read
+                // one step ahead; the raw fp8 bytes are the A operand.
+                auto key = [&](int i) {
+                    const uint32_t at = ko ^ ((i & 3) * 128) ^ (sa_swz(16 * (i >> 2)) * 16);
+                    const v4i x = *(LdsV4i)(at + (i >> 2) * 16 * kValueDim);
+                    const v4i y = *(LdsV4i)((at ^ 64) + (i >> 2) * 16 * kValueDim);
+                    return v8i{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+                };
+                auto logits = [&](auto&& dot) {
+                    v8i kv[2] = {key(0), v8i{}};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int u = i >> 2, g = i & 3;
-                const f32x4 s4 = *(LdsF32x4)(sl + (g * kSaTile + 16 * u) * 4);
-                if (i + 1 < 8) kv[(i + 1) & 1] = key(i + 1);
-                __builtin_amdgcn_sched_barrier(0);
-                f32x4 part = sa_mma8(kv[i & 1], qh[g], f32x4{0.f, 0.f, 0.f, 0.f}, g, qscale);
-                part = sa_mma8(kv[i & 1], ql[g], part, g, qscale);
+                    for (int i = 0; i < 8; ++i) {
+                        const int u = i >> 2, g = i & 3;
+                        const f32x4 s4 = *(LdsF32x4)(sl + (g * kSaTile + 16 * u) * 4);
+                        if (i + 1 < 8) kv[(i + 1) & 1] = key(i + 1);
+                        __builtin_amdgcn_sched_barrier(0);
+                        const f32x4 part = dot(kv[i & 1], g);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sv[u][e] = fmaf(part[e], s4[e], sv[u][e]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // Softmax: pr = 2^(logit - m), the logits of tokens without a row at -inf.
-            float pr[8];
-            float mx = -INFINITY;
+                        for (int e = 0; e < 4; ++e) sv[u][e] = fmaf(part[e], s4[e], sv[u][e]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                };
+                if constexpr (!kWide) {
+                    logits([&](v8i k, int g) {
+                        const f32x4 part = sa_mma8(k, qh[g], f32x4{0.f, 0.f, 0.f, 0.f}, g, qscale);
+                        return sa_mma8(k, ql[g], part, g, qscale_lo);
+                    });
+                } else {
+                    logits([&](v8i k, int g) {
+                        f32x4 part = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) pr[i] = sv[i >> 2][i & 3] * scale2;
-            if (mask != kAll) {
-                const uint32_t mine = mask >> (4 * tk);
+                        for (int x = 0; x < 4; ++x) {
+                            const v8i& q = x < 2 ? qh[g] : ql[g];
+                            const v4i qx = {q[4 * (x & 1)], q[4 * (x & 1) + 1], q[4 * (x & 1) + 2], q[4 * (x & 1) + 3]};
+                            part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16(k[2 * x], k[2 * x + 1]),
+                                                                           __builtin_bit_cast(bf16x8, qx), part, 0, 0, 0);
+                        }
+                        return part;
+                    });
+                }
+                // Softmax: pr = 2^(logit - m), the logits of tokens without a row at -inf.
+                float pr[8];
+                float mx = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) pr[i] = sv[i >> 2][i & 3] * scale2;
+                if (mask != kAll) {
+                    const uint32_t mine = mask >> (4 * tk);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if (!((mine >> (16 * (i >> 2) + (i & 3))) & 1u)) pr[i] = -INFINITY;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) mx = fmaxf(mx, pr[i]);
+                mx = rows4_max(mx);
+                const bool raise = mx > m_run + kSaMargin;  // also the first finite maximum
+                if (__ballot(raise) != 0ull) {
+                    const float m_new = raise ? mx : m_run;
+                    const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+                    const float a = raise ? alpha : 1.f;
+                    l_sum *= a;
+#pragma unroll
+                    for (int t = 0; t < kBlocks; ++t) o[t] *= a;
+                    m_run = m_new;
+                }
+                const float bias = m_run == -INFINITY ? 0.f : -m_run;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    if (!((mine >> (16 * (i >> 2) + (i & 3))) & 1u)) pr[i] = -INFINITY;
+                    pr[i] = __builtin_amdgcn_exp2f(pr[i] + bias);
+                    l_sum += pr[i];
                 }
-            }
+                // Value product [features, heads]: the transpose loads of kAhead blocks ahead of the MFMAs
+                // of the kAhead before them; each scale group's probabilities as its first block comes up.
+                constexpr int kAhead = G == 1 ? 4 : 2;  // two waves per SIMD have no registers for more
+                auto value = [&](int t) {
+                    return __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsI32x2)((vo ^ ((t & 15) * 16)) + (t & 16) * 16));
+                };
+                i32x2 raw[2][kAhead];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) mx = fmaxf(mx, pr[i]);
-            mx = rows4_max(mx);
-            const bool raise = mx > m_run + kSaMargin;  // also the first finite maximum
-            if (__ballot(raise) != 0ull) {
-                const float m_new = raise ? mx : m_run;
-                const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
-                const float a = raise ? alpha : 1.f;
-                l_sum *= a;
+                for (int i = 0; i < kAhead; ++i) raw[0][i] = value(i);
+                bf16x8 pb;
 #pragma unroll
-                for (int t = 0; t < kBlocks; ++t) o[t] *= a;
-                m_run = m_new;
-            }
-            const float bias = m_run == -INFINITY ? 0.f : -m_run;
+                for (int t = 0; t < kBlocks; t += kAhead) {
+                    const int now = t / kAhead & 1;
+                    if (t + kAhead < kBlocks) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                pr[i] = __builtin_amdgcn_exp2f(pr[i] + bias);
-                l_sum += pr[i];
-            }
-            // Value product [features, heads]: the transpose loads of kAhead blocks ahead of the MFMAs
-            // of the kAhead before them; each scale group's probabilities as its first block comes up.
-            constexpr int kAhead = G == 1 ? 4 : 2;  // two waves per SIMD have no registers for more
-            auto value = [&](int t) {
-                return __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsI32x2)((vo ^ ((t & 15) * 16)) + (t & 16) * 16));
-            };
-            i32x2 raw[2][kAhead];
-#pragma unroll
-            for (int i = 0; i < kAhead; ++i) raw[0][i] = value(i);
-            bf16x8 pb;
-#pragma unroll
-            for (int t = 0; t < kBlocks; t += kAhead) {
-                const int now = t / kAhead & 1;
-                if (t + kAhead < kBlocks) {
-#pragma unroll
-                    for (int i = 0; i < kAhead; ++i) raw[now ^ 1][i] = value(t + kAhead + i);
-                }
-                if (t % 8 == 0) {
-                    v4i packed;
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        const f32x4 s4 = *(LdsF32x4)(sl + (t / 8 * kSaTile + 16 * u) * 4);
-                        packed[2 * u] = static_cast<int>(pack_bf16(pr[4 * u] * s4[0], pr[4 * u + 1] * s4[1]));
-                        packed[2 * u + 1] = static_cast<int>(pack_bf16(pr[4 * u + 2] * s4[2], pr[4 * u + 3] * s4[3]));
+                        for (int i = 0; i < kAhead; ++i) raw[now ^ 1][i] = value(t + kAhead + i);
                     }
-                    pb = __builtin_bit_cast(bf16x8, packed);
-                }
-                __builtin_amdgcn_sched_barrier(0);
+                    if (t % 8 == 0) {
+                        v4i packed;
 #pragma unroll
-                for (int i = 0; i < kAhead; ++i) {
-                    const i32x2 x = raw[now][i];
-                    o[t + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16(x[0], x[1]), pb, o[t + i], 0, 0, 0);
+                        for (int u = 0; u < 2; ++u) {
+                            const f32x4 s4 = *(LdsF32x4)(sl + (t / 8 * kSaTile + 16 * u) * 4);
+                            packed[2 * u] = static_cast<int>(pack_bf16(pr[4 * u] * s4[0], pr[4 * u + 1] * s4[1]));
+                            packed[2 * u + 1] = static_cast<int>(pack_bf16(pr[4 * u + 2] * s4[2], pr[4 * u + 3] * s4[3]));
+                        }
+                        pb = __builtin_bit_cast(bf16x8, packed);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < kAhead; ++i) {
+                        const i32x2 x = raw[now][i];
+                        o[t + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16(x[0], x[1]), pb, o[t + i], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
+            mask = next;
         }
-        mask = next;
-    }
+    };
+    if (!wide) stream(std::false_type{});
+    else stream(std::true_type{});
 
     // Merge of the streams: with the maximum M over them, out = sum_w 2^(m_w - M) o_w / l and
     // l = sum_w 2^(m_w - M) l_w, 512 / G features at a time through LDS.
+    const int le = fresh(lane), mn = le & 15, mk = le >> 4;  // n and kg, not held over the tiles
     const float l_all = rows4_sum(l_sum);
     float* s_m = reinterpret_cast<float*>(s_mem + kLdsScale);  // [wave][head], then the sums
     float* s_f = s_m + 2 * kWaves * kSaHeads;                  // [wave][head]: factor of the wave's output
@@ -527,16 +603,16 @@ __global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kerne
     constexpr int kPitch = kValueDim / G + 4;
     static_assert(kWaves * kSaHeads * kPitch * 4 <= kLdsScale, "merge buffer inside ring and rope");
     __syncthreads();  // every wave is done with its ring, rope and scales
-    if (kg == 0) {
-        s_m[w * kSaHeads + n] = m_run;
-        s_m[(kWaves + w) * kSaHeads + n] = l_all;
+    if (mk == 0) {
+        s_m[w * kSaHeads + mn] = m_run;
+        s_m[(kWaves + w) * kSaHeads + mn] = l_all;
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         if (g > 0) __syncthreads();  // the features before have been read
 #pragma unroll
         for (int t = 0; t < kBlocks / G; ++t) {
-            *reinterpret_cast<f32x4*>(buf + (w * kSaHeads + n) * kPitch + t * 16 + 4 * kg) = o[g * (kBlocks / G) + t];
+            *reinterpret_cast<f32x4*>(buf + (w * kSaHeads + mn) * kPitch + t * 16 + 4 * mk) = o[g * (kBlocks / G) + t];
         }
         __syncthreads();
         if (g == 0) {

@@ -265,3 +265,80 @@ def test_sparse_attention_edges_against_64_bits(torch_gpu, heads, rows, per_requ
         worst = max(worst, ((out[r] - want).abs() / bound).max().item())
     say(f"  worst error over its bound: {worst:.3f}")
     assert worst <= 1.0
+
+
+@pytest.mark.parametrize("heads,rows,spread", [
+    (16, 3, "span"), (40, 5, "span"), (128, 64, "span"), (16, 3, 10), (16, 64, 14), (40, 5, 12), (40, 5, 20),
+    (128, 64, 16), (8, 200, 60)])
+def test_sparse_attention_query_spread_against_64_bits(torch_gpu, heads, rows, spread):
+    """Queries whose large features meet zero key bytes, so that the logits are made of the small ones.
+    "span": features down to 2^-13 of their scale group's largest, the bytes zero at those above
+    2^-6. A number k: one feature of groups 0 and 2 of the first 16 heads is 2^k times the
+    others and meets zero bytes. The logits are scaled to a standard deviation of 3, so an error in
+    them shows in the output. The bound is that of the test above: one bf16 rounding per
+    probability, doubled."""
+    torch = torch_gpu
+    gen = torch.Generator(device="cuda").manual_seed(heads * 100 + rows)
+    blocks, max_blocks = 64, 20
+    q = torch.randn((rows, heads, 576), generator=gen, device="cuda")
+    codes = (torch.randn((blocks * 128, 4, 128), generator=gen, device="cuda") * 60).to(torch.float8_e4m3fn)
+    if spread == "span":
+        at = torch.arange(512, device="cuda") % 14  # power of two below the largest
+        q[:, :, :512] = (1 + torch.rand((rows, heads, 512), generator=gen, device="cuda")) * torch.exp2(6.0 - at)
+        q[:, :, :512] *= torch.where(torch.rand((rows, heads, 512), generator=gen, device="cuda") < 0.5, -1.0, 1.0)
+        q = torch.where(q.to(torch.bfloat16).abs() >= 128, 127.5, q)  # no value rounds into the next power of two
+        codes.view(torch.uint8).view(-1, 512)[:, at < 6] = 0
+    else:
+        for feature in (17, 300):
+            q[:, :16, feature] = 1.37 * 2.0 ** spread
+            codes.view(torch.uint8).view(-1, 512)[:, feature] = 0
+    q = q.to(torch.bfloat16)
+    scales = torch.rand((blocks * 128, 4), generator=gen, device="cuda") * 0.01 + 0.01
+    rope = torch.randn((blocks * 128, 64), generator=gen, device="cuda").to(torch.bfloat16)
+    kv = torch.empty((blocks * 128, ROW), dtype=torch.uint8, device="cuda")
+    kv[:, :512] = codes.view(torch.uint8).view(-1, 512)
+    kv[:, 512:640] = rope.view(torch.uint8)
+    kv[:, 640:] = scales.view(torch.uint8)
+    table = torch.stack([torch.randperm(blocks, generator=gen, device="cuda")[:max_blocks] for _ in range(rows)])
+    table = table.to(torch.int32)
+    idx = torch.randint(0, max_blocks * 128, (rows, TOPK), generator=gen, device="cuda", dtype=torch.int32)
+    key = torch.cat([(codes.double() * scales.double()[:, :, None]).view(-1, 512), rope.double()], dim=1)
+    picked = {r: key[table[r].long()[idx[r].long() // 128] * 128 + idx[r].long() % 128].contiguous()
+              for r in sorted({0, rows // 2, rows - 1})}
+    scale = 3.0 / (q[0].double() @ picked[0].T.contiguous()).std().item()
+    say(f"case query spread heads={heads} rows={rows} spread={spread} scale={scale:.4f}")
+    out = sparse_attention(q, kv.view(blocks, 128, ROW), table, idx, scale).double()
+    worst = 0.0
+    for r, k in picked.items():
+        prob = torch.softmax(q[r].double() @ k.T.contiguous() * scale, dim=1)
+        bound = 2.0 ** -8 * (prob @ k[:, :512].abs().contiguous()) + 1e-7
+        worst = max(worst, ((out[r] - prob @ k[:, :512].contiguous()).abs() / bound).max().item())
+    say(f"  worst error over its bound: {worst:.3f}")
+    assert worst <= 1.0
+
+
+@pytest.mark.parametrize("heads", [16, 40])
+def test_sparse_attention_nonfinite_query_stays_in_its_head(torch_gpu, heads):
+    """A NaN feature makes its head NaN. An infinite one that meets only negative key bytes makes every
+    logit of its head -inf, and that head is zero. The other heads are as without them."""
+    torch = torch_gpu
+    gen = torch.Generator(device="cuda").manual_seed(heads)
+    rows, blocks = 2, 32
+    kv = torch.zeros((blocks * 128, ROW), dtype=torch.uint8, device="cuda")
+    codes = (torch.randn((blocks * 128, 512), generator=gen, device="cuda") * 60).to(torch.float8_e4m3fn)
+    codes.view(torch.uint8)[:, 200] = 0xB8  # -1
+    kv[:, :512] = codes.view(torch.uint8)
+    kv[:, 640:] = torch.full((4,), 0.02, device="cuda").view(torch.uint8)
+    table = torch.arange(blocks, dtype=torch.int32, device="cuda").expand(rows, blocks).contiguous()
+    idx = torch.randint(0, blocks * 128, (rows, TOPK), generator=gen, device="cuda", dtype=torch.int32)
+    q = torch.randn((rows, heads, 576), generator=gen, device="cuda").to(torch.bfloat16)
+    say(f"case nonfinite query heads={heads}")
+    want = sparse_attention(q, kv.view(blocks, 128, ROW), table, idx, SCALE).clone()
+    q[:, 3, 5], q[:, 4, 200] = float("nan"), float("inf")
+    out = sparse_attention(q, kv.view(blocks, 128, ROW), table, idx, SCALE)
+    say("  infinite head:", out[:, 4].unique()[:4].tolist())
+    assert out[:, 3].isnan().all() and (out[:, 4] == 0).all()
+    others = [h for h in range(heads) if h not in (3, 4)]
+    err = (out[:, others] - want[:, others]).abs().max().item()
+    say(f"  other heads: max abs difference {err:.2e}")
+    assert err <= 2.0 ** -8 * 448 * 0.02 / 4  # p rounded once to bf16, |v| mostly far below its largest
