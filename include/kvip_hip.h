@@ -629,8 +629,8 @@ uint32_t kvip_hip_lifetch_plan(const KvipLIFetchArgs* args);
 #define KVIP_LIFETCH_STATIC_SCRATCH_BYTES (16u << 20)
 uint32_t kvip_hip_lifetch_forward_static(const KvipLIFetchArgs* args, void* stream);
 /* TopK-2048 of rows scored by kvip_hip_indexer_decode fused with the Fetch gather of the
- * selected rows: same outputs as kvip_hip_topk followed by kvip_hip_fetch_gather. Needs
- * topk->histogram and topk->segments; fetch->topk must be topk->topk. */
+ * selected rows: same outputs as kvip_hip_topk followed by kvip_hip_fetch_gather, the errors of
+ * both in topk->status. Needs topk->histogram and topk->segments; fetch->topk must be topk->topk. */
 uint32_t kvip_hip_select_fetch(const KvipTopkArgs* topk, const KvipFetchArgs* fetch, void* stream);
 uint32_t kvip_hip_update_abc(const KvipAbcArgs* args, void* stream);
 uint32_t kvip_hip_lru_reset(const KvipLruArgs* args, int32_t committed, void* stream);

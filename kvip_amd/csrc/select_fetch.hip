@@ -133,7 +133,7 @@ __global__ __launch_bounds__(THREADS) void select_gather_kernel(const KvipTopkAr
     const size_t segs = (static_cast<size_t>(p.key_stride) + KVIP_TOPK_SEGMENT_KEYS - 1) / KVIP_TOPK_SEGMENT_KEYS;
     uint32_t* tickets = p.segments + static_cast<size_t>(row) * segs * KVIP_TOPK_SEGMENT_WORDS + kTicketWord;
     uint32_t ticket = 0;
-    uint32_t err = 0;
+    uint32_t err = 0, gather_err = 0;
 
     if (valid < kTopK) {
         // Short row: every token in order, then -1 (zero rows).
@@ -190,7 +190,10 @@ __global__ __launch_bounds__(THREADS) void select_gather_kernel(const KvipTopkAr
     // TopK output of this part (coalesced), then the gather.
     for (int i = tid; i < part_rows; i += THREADS) out[pos0 + i] = s_tok[i];
 #pragma unroll 1
-    for (int e0 = wave * ROWS; e0 < part_rows; e0 += kWaves * ROWS) gather_pass<ROWS, PIECES>(f, b, out_rows, s_tok, e0, err);
+    for (int e0 = wave * ROWS; e0 < part_rows; e0 += kWaves * ROWS) {
+        gather_pass<ROWS, PIECES>(f, b, out_rows, s_tok, e0, gather_err);
+    }
+    report(f.status, gather_err);
     report(p.status, err);
 }
 
@@ -232,6 +235,7 @@ uint32_t validate_select_fetch(const KvipTopkArgs* t, const KvipFetchArgs* f) {
     return ok ? KVIP_OK : KVIP_ERR_INVALID;
 }
 
+// Histogram errors go to t.status and the gather's to f.status, as from the two separate launches.
 hipError_t launch_select_fetch(const KvipTopkArgs& t, const KvipFetchArgs& f, hipStream_t stream) {
     return f.row_bytes == KVIP_KV_ROW_BYTES ? launch_pieces<KVIP_KV_ROW_BYTES / 16>(t, f, stream)
                                             : launch_pieces<0>(t, f, stream);
@@ -243,5 +247,7 @@ extern "C" uint32_t kvip_hip_select_fetch(const KvipTopkArgs* topk, const KvipFe
     if (topk == nullptr || fetch == nullptr) return KVIP_ERR_INVALID;
     const uint32_t rc = kvip::validate_select_fetch(topk, fetch);
     if (rc != KVIP_OK) return rc;
-    return static_cast<uint32_t>(kvip::launch_select_fetch(*topk, *fetch, static_cast<hipStream_t>(stream)));
+    KvipFetchArgs f = *fetch;
+    f.status = topk->status;  // this entry point reports everything in one word
+    return static_cast<uint32_t>(kvip::launch_select_fetch(*topk, f, static_cast<hipStream_t>(stream)));
 }

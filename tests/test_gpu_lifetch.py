@@ -498,3 +498,40 @@ def test_topk_of_long_rows_on_wide_segments(torch_gpu, kind, ctx):
             assert np.array_equal(got[r], ref.topk_reference(keys[r], v)), f"row {r} valid {v}"
         assert int(rot.status.item()) == 0
         assert not rot.histogram.any() and not rot.topk_segments[:, 0, -1].any()
+
+
+@pytest.mark.parametrize("batch,split", [(1, True), (4, True), (16, True), (17, True), (4, False)])
+def test_forward_reports_the_gathers_errors_to_its_own_status(torch_gpu, batch, split):
+    """A block id that is bad in the Fetch's table only, one status word per stage: the forward sets
+    the Fetch's word and no other, whether the gather is fused with the TopK (up to 16 query
+    rows with work memory) or a launch of its own; the rows of the bad block are zeros. The fused
+    launch called by itself sets the TopK's word."""
+    torch = torch_gpu
+    say(f"case status words batch={batch} split={split}")
+    wl = synthetic.decode_workload(torch, batch=batch, ctx=[3000] * (batch - 1) + [2047], device="cuda", seed=batch)
+    rot, upd, fwd = synthetic.bind(torch, kvip_amd, wl)
+    table = rot.block_table.clone()
+    table[batch - 1, 3] = rot.num_blocks + 5
+    words = torch.zeros(3, dtype=torch.int32, device="cuda")
+
+    def run(entry, *args):
+        words.zero_()
+        assert entry(*args, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return words.tolist()
+
+    indexer, topk, fetch = rot.indexer_args(), rot.topk_args(split=split), upd.fetch_args()
+    fetch.block_table = table.data_ptr()
+    indexer.status, topk.status, fetch.status = (words[i:].data_ptr() for i in range(3))
+    args = abi.LIFetchArgs(indexer, topk, fetch)
+    assert run(fwd.library.kvip_hip_lifetch_forward, ctypes.byref(args)) == [0, 0, abi.STATUS_BAD_BLOCK]
+    rows = upd.output[batch - 1].any(1)  # of the 2047 tokens in order, then an empty one
+    assert not rows[384:512].any() and not rows[2047] and rows[:384].all() and rows[512:2047].all()
+    topk.status = 0
+    args = abi.LIFetchArgs(indexer, topk, fetch)
+    assert run(fwd.library.kvip_hip_lifetch_forward, ctypes.byref(args)) == [0, 0, abi.STATUS_BAD_BLOCK]
+    if split:
+        topk.status = words[1:].data_ptr()
+        fwd.score()
+        assert run(fwd.library.kvip_hip_select_fetch, ctypes.byref(topk), ctypes.byref(fetch)) == \
+            [0, abi.STATUS_BAD_BLOCK, 0]
