@@ -50,13 +50,18 @@ typedef __attribute__((address_space(3))) uint32_t* LdsU32;
 // lds + lane * 16 (4), lds wave-uniform. The wait insertion does not see them, so LDS accesses
 // stay ordinary code that the compiler schedules and waits for exactly; the kernel waits for the
 // loads themselves with an explicit vmcnt. They have no output registers, so nothing can be
-// reused while they are in flight; kernels using them must not use m0 otherwise.
+// reused while they are in flight. m0 is named as clobbered, so that the compiler sets it anew for
+// its own uses (the direct-to-LDS builtin among them); the diagnostic that it is a reserved register
+// means only that asm cannot preserve its value.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 KVIP_DEVICE void dma16(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
 }
 KVIP_DEVICE void dma4(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds), "v"(src) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 KVIP_DEVICE uint32_t lds_read_b32(uint32_t a) {
     uint32_t v;
