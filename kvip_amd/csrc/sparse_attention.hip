@@ -60,6 +60,10 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
+// Output and workspace are float arrays of any alignment (the card takes 16-byte accesses at
+// 4-byte addresses).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2_any __attribute__((ext_vector_type(2), aligned(4)));
 
 constexpr int kSaHeads = 16;                // heads per wave (MFMA N)
 constexpr int kSaStreams = 4;               // token streams per workgroup
@@ -659,7 +663,7 @@ __global__ __launch_bounds__(kSaStreams * G * 64, 1) void sparse_attention_kerne
             if (h < p.heads) {
                 const size_t rh = static_cast<size_t>(r) * p.heads + h;
                 float* out = splits == 1 ? p.output + rh * kValueDim : p.workspace + (rh * splits + sp) * kValueDim;
-                *reinterpret_cast<f32x4*>(out + g * (kValueDim / G) + f) = v;
+                *reinterpret_cast<f32x4_any*>(out + g * (kValueDim / G) + f) = v;
             }
         }
     }
@@ -677,9 +681,9 @@ __global__ __launch_bounds__(256) void sparse_attention_merge_kernel(const KvipS
     f32x4 part[SPLITS];
     f32x2 sums[SPLITS];
 #pragma unroll
-    for (int s = 0; s < SPLITS; ++s) sums[s] = *reinterpret_cast<const f32x2*>(ml + 2 * s);
+    for (int s = 0; s < SPLITS; ++s) sums[s] = *reinterpret_cast<const f32x2_any*>(ml + 2 * s);
 #pragma unroll
-    for (int s = 0; s < SPLITS; ++s) part[s] = *reinterpret_cast<const f32x4*>(ws + s * kValueDim);
+    for (int s = 0; s < SPLITS; ++s) part[s] = *reinterpret_cast<const f32x4_any*>(ws + s * kValueDim);
     float m = -INFINITY;
 #pragma unroll
     for (int s = 0; s < SPLITS; ++s) m = fmaxf(m, sums[s][0]);
@@ -691,7 +695,7 @@ __global__ __launch_bounds__(256) void sparse_attention_merge_kernel(const KvipS
         l += wgt * sums[s][1];
         v += wgt * part[s];
     }
-    *reinterpret_cast<f32x4*>(p.output + rh * kValueDim + f) = v * (l > 0.f ? 1.f / l : 0.f);
+    *reinterpret_cast<f32x4_any*>(p.output + rh * kValueDim + f) = v * (l > 0.f ? 1.f / l : 0.f);
 }
 
 template <int SPLITS>

@@ -12,12 +12,15 @@ rows at 128 heads, whose workgroups write the normalised output themselves), the
 buffer of the contiguous LIFetch forward, and the resident hot cache addressed by the slot
 outputs (the reference's check_sfa flow: slots from the round, values from the logical
 tokens' payload)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import kvip_amd
 from kvip_amd import synthetic
 from kvip_amd.operators.sfa import gathered_table, hot_cache_table, sparse_attention
+from kvip_amd.runtime import abi
 from oracle import sfa
 
 pytestmark = pytest.mark.gpu
@@ -342,3 +345,30 @@ def test_sparse_attention_nonfinite_query_stays_in_its_head(torch_gpu, heads):
     err = (out[:, others] - want[:, others]).abs().max().item()
     say(f"  other heads: max abs difference {err:.2e}")
     assert err <= 2.0 ** -8 * 448 * 0.02 / 4  # p rounded once to bf16, |v| mostly far below its largest
+
+
+@pytest.mark.parametrize("rows,heads", [(2, 16), (3, 40), (260, 16)])
+def test_sparse_attention_buffers_of_any_float_alignment(torch_gpu, rows, heads):
+    """Output and workspace (16 splits for few rows, none for 260) 4 bytes past a 16-byte boundary: the
+    same output, bit for bit, and nothing written beside it."""
+    torch = torch_gpu
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    blocks = 24
+    kv = torch.zeros((blocks, 128, ROW), dtype=torch.uint8, device="cuda")
+    kv[:, :, :512] = torch.randint(0, 120, (blocks, 128, 512), generator=gen, device="cuda", dtype=torch.uint8)
+    kv[:, :, 640:] = torch.full((4,), 0.01, device="cuda").view(torch.uint8)
+    table = torch.arange(blocks, dtype=torch.int32, device="cuda").expand(rows, blocks).contiguous()
+    idx = torch.randint(0, blocks * 128, (rows, TOPK), generator=gen, device="cuda", dtype=torch.int32)
+    q = torch.randn((rows, heads, 576), generator=gen, device="cuda").to(torch.bfloat16)
+    op = kvip_amd.SparseAttention(torch, rows=rows, heads=heads, device="cuda").bind(q, kv, table, idx)
+    say(f"case float alignment rows={rows} heads={heads}")
+    want = op().clone()
+    out = torch.full((want.numel() + 8,), 7.0, device="cuda")
+    work = torch.empty(op.workspace.numel() + 4, device="cuda")
+    args = abi.SparseAttnArgs.from_buffer_copy(op.args)
+    args.output, args.workspace = out[1:].data_ptr(), work[1:].data_ptr()
+    assert args.output % 16 == 4 and args.workspace % 16 == 4
+    assert op.library.kvip_hip_sparse_attention(ctypes.byref(args), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out[1:1 + want.numel()].view_as(want), want)
+    assert out[0] == 7 and (out[1 + want.numel():] == 7).all()
