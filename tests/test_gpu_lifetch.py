@@ -535,3 +535,28 @@ def test_forward_reports_the_gathers_errors_to_its_own_status(torch_gpu, batch, 
         fwd.score()
         assert run(fwd.library.kvip_hip_select_fetch, ctypes.byref(topk), ctypes.byref(fetch)) == \
             [0, abi.STATUS_BAD_BLOCK, 0]
+
+
+@pytest.mark.parametrize("qk,batch,rpr,ctx,split,launches", [
+    ("fp8", 1, 1, 100, True, 2), ("fp8", 16, 1, 8192, True, 2), ("bf16", 4, 4, 32768, True, 2),
+    ("fp8", 17, 1, 8192, True, 3), ("bf16", 9, 2, 8192, True, 3), ("fp8", 2, 1, 32769, True, 3),
+    ("fp8", 2, 1, 65537, True, 4), ("fp8", 16, 1, 8192, False, 3)])
+def test_forward_launch_count(torch_gpu, qk, batch, rpr, ctx, split, launches):
+    """The kernels of one captured forward: two up to 16 query rows of 32768 keys with work memory (TopK
+    fused with the gather), three above or without it, four above 65536 keys (split select)."""
+    torch = torch_gpu
+    say(f"case launch count {qk} batch={batch} rpr={rpr} ctx={ctx} split={split}")
+    wl = synthetic.decode_workload(torch, batch=batch, ctx=[ctx] * batch, device="cuda", qk=qk,
+                                   key_scale=qk == "fp8", rows_per_request=rpr, seed=3)
+    rot, upd, fwd = synthetic.bind(torch, kvip_amd, wl)
+    args = abi.LIFetchArgs(rot.indexer_args(), rot.topk_args(split=split), upd.fetch_args())
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        assert fwd.library.kvip_hip_lifetch_forward(ctypes.byref(args), torch.cuda.current_stream().cuda_stream) == 0
+    count = ctypes.c_size_t()
+    assert fwd.library.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    assert count.value == launches
+    graph.instantiate()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert int(rot.status.item()) == 0
