@@ -219,9 +219,9 @@ typedef struct KvipFetchArgs {
     int32_t num_blocks;
 } KvipFetchArgs;
 
-/* One decode round: scoring -> TopK-2048 -> Fetch gather, stream-ordered (three
- * launches; the stages must be chained: TopK reads the scoring's keys and histogram, the
- * gather the TopK's ids). */
+/* One decode round: scoring -> TopK-2048 -> Fetch gather, stream-ordered (two to four launches,
+ * kvip_hip_lifetch_plan; the stages must be chained: TopK reads the scoring's keys and
+ * histogram, the gather the TopK's ids). */
 typedef struct KvipLIFetchArgs {
     KvipIndexerArgs indexer;
     KvipTopkArgs topk;
@@ -542,7 +542,10 @@ typedef struct KvipPageArgs {
  * b = r / rows_per_request) and head h, over j with indices[r][j] >= 0 (position t lives in
  * block block_table[b][t / 128], row t % 128, of kv_cache):
  *   s_j = scale * <query[r][h], key_j>, p_j = exp(s_j - max s),
- *   output[r][h] = sum_j bf16(p_j) * value_j / sum_j p_j   (0 when no index is valid).
+ *   output[r][h] = sum_j p_j * value_j / sum_j p_j   (0 when no index is valid),
+ * where p_j times a group's scale is rounded once to bf16 and multiplies the group's nope features;
+ * everything else is exact or fp32 (query features more than 2^14 below the largest of their 128
+ * may be off by 2^-22 of it).
  * Bad positions or blocks set KVIP_STATUS_BAD_TOKEN / _BAD_BLOCK and count as absent. */
 typedef struct KvipSparseAttnArgs {
     const uint16_t* query;        /* [rows, heads, 576] bf16, 16-byte aligned */
@@ -608,11 +611,12 @@ uint32_t kvip_hip_indexer_prefill(const KvipPrefillArgs* args, void* stream);
 uint32_t kvip_hip_indexer_prefill_grid(const KvipPrefillArgs* args, int32_t workgroups, void* stream);
 uint32_t kvip_hip_lifetch_forward(const KvipLIFetchArgs* args, void* stream);
 /* The launch plan kvip_hip_lifetch_forward takes for these arguments (no launch, no device
- * access): KVIP_LIFETCH_PLAN_THREE (scoring, TopK, gather; rows of at most
+ * access): KVIP_LIFETCH_PLAN_THREE (the three stages scoring, TopK, gather; rows of at most
  * KVIP_TOPK_REGS_MAX_KEYS keys use the register-resident TopK; up to 16 query rows of at most
  * 32768 keys with topk.segments given run TopK and gather as one launch), or KVIP_ERR_INVALID when
  * the forward would reject them. A host query with no counterpart in the reference, for
- * callers and tests that need to know which kernels a round runs. */
+ * callers and tests that need to know how a round runs; how many launches the three stages take
+ * follows from the sizes as stated, not from the code returned. */
 #define KVIP_LIFETCH_PLAN_THREE 0u
 #define KVIP_TOPK_REGS_MAX_KEYS 65536
 uint32_t kvip_hip_lifetch_plan(const KvipLIFetchArgs* args);

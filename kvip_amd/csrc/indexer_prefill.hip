@@ -30,9 +30,9 @@
 // per SIMD spills and is twice as slow. What could be trimmed is around the loop: both rows (bf16:
 // both tiles) are joined by one lane swap, the key comes straight from the rounded 32-bit pattern,
 // the next tile's fragments are requested under the epilogue, and bf16 chunks are as long as fp8
-// ones, with half the barriers they had at 128 tokens. Scoring 4096 rows causally against 65536
-// keys in fp8 went from 1948 to 1905 us, six sequences of up to 900 rows against up to 9000 keys
-// from 150 to 142 us, 2048 rows against 16384 keys in bf16 from 462 to 454 us.
+// ones, with half the barriers they had at 128 tokens. With 4096 keys per item on either side, scoring
+// 4096 rows causally against 65536 keys went from 1917 to 1881 us in fp8 and 3640 to 3485 in bf16, 2048
+// rows against 16384 keys from 251 to 246 and 458 to 440.
 //
 // Reference: the native prefill LI (torch_npu.npu_quant_lightning_indexer, TND layout,
 // sparse_mode 3) that the vLLM selector runs for prefill rows (python/kvip/adapters/vllm/
@@ -464,13 +464,13 @@ int64_t prefill_items(const KvipPrefillArgs& a, int segment) {
 // shapes of 16 to 8192 rows against 1024 to 65536 keys: lead 0.5 and tail 1 for fp8, 1.25 and
 // 0.25 for bf16 (twice the Q, one workgroup per CU); the choice is within 1% (fp8) and 3% (bf16) of
 // the best segment on average, 19% at worst. Against 4096 keys throughout, scoring alone, us fp8 /
-// bf16: 16 rows x 4096 keys 84.6 -> 11.7 / 100.6 -> 13.8, 64 x 16384 86.3 -> 24.0 / 102.8 -> 41.7, 512 x
-// 8192 88.0 -> 49.8 / 104.2 -> 66.8, six sequences of 33-900 rows 125 -> 106 / 199 -> 190, 4096 x 16384
-// 497 -> 466 / 886 -> 854. Long segments stay where items are many: 2048 x 65536 takes 974 us with
-// 4096 keys and 1447 with 256. A bounded grid keeps 4096 keys: its launch runs beside other kernels,
-// which take the CUs of the workgroups that run out of items, and items of equal size would hold all
-// of them to the end (a round of 32 decode requests beside chunks of 2048 x 8192 and 1536 x 1536:
-// 307-310 us with short segments, 276-279 with these).
+// bf16: 16 rows x 4096 keys 79.2 -> 12.3 / 90.0 -> 14.5, 64 x 16384 79.8 -> 24.5 / 92.3 -> 41.5, 512 x
+// 8192 80.9 -> 45.9 / 97.2 -> 63.7, six sequences of 33-900 rows against 900-9000 keys 140 -> 120 / 206
+// (the same), 4096 x 16384 477 -> 450 / 817 (the same). Long segments stay where items are many:
+// 2048 x 65536 takes 974 us with 4096 keys and 1447 with 256. A bounded grid keeps 4096 keys: its
+// launch runs beside other kernels, which take the CUs of the workgroups that run out of items, and
+// items of equal size would hold all of them to the end (a round of 32 decode requests beside
+// chunks of 2048 x 8192 and 1536 x 1536: 307-310 us with short segments, 276-279 with these).
 int prefill_segment(const KvipPrefillArgs& a, int workgroups) {
     if (workgroups > 0) return kPfSegment;
     constexpr int64_t cus = 256;

@@ -167,8 +167,9 @@ __global__ __launch_bounds__(THREADS) void select_gather_kernel(const KvipTopkAr
         uint32_t gt_hi;
         wave_select_bin(h, kTopK, hb, gt_hi);
         __syncthreads();
-        // Every wave of this part has read the histogram: take the row's ticket now, so that its
-        // round trip passes under the selection.
+        // Every wave of this part has read the histogram: take the row's ticket now and not after the
+        // gather, which would end with its round trip. The compiler has wave 0 wait for the reply at
+        // once; the other waves go on to the selection's first barrier.
         if (tid == 0) ticket = __hip_atomic_fetch_add(tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // Steps 2-4: the tokens whose positions fall in this part's share go to s_tok.
         const RowSelection sel = select_row<KPT>(kk, count, first, hb, gt_hi, s_hist, s_wave, [&](int pos, int tok) {
@@ -178,7 +179,9 @@ __global__ __launch_bounds__(THREADS) void select_gather_kernel(const KvipTopkAr
         // The scoring histogram counts every visible key once: another total means the scoring
         // launch skipped or repeated tiles.
         const uint32_t counted = wave_inclusive_scan(h[0] + h[1] + h[2] + h[3]);
-        if (part == 0 && tid == 63 && !(sel.ok && counted == static_cast<uint32_t>(valid))) err |= KVIP_STATUS_HISTOGRAM;
+        if (part == 0 && tid == 63 && !(sel.ok && counted == static_cast<uint32_t>(valid))) {
+            err |= KVIP_STATUS_HISTOGRAM;
+        }
     }
     // The part holding the last ticket clears the histogram for the next scoring launch.
     if (tid == 0) s_last = valid >= kTopK && ticket == static_cast<uint32_t>(parts) - 1u;

@@ -131,7 +131,8 @@ class LIFetchForward:
 
     @property
     def plan(self):
-        """The launch plan of a contiguous-Fetch forward: "three" (scoring, TopK, gather);
+        """The launch plan of a contiguous-Fetch forward: "three" (the stages scoring, TopK, gather,
+        of which the last two are one launch up to 16 query rows of at most 32768 keys);
         "resident" for the resident-cache forward."""
         if self.resident:
             return "resident"
