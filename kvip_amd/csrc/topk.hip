@@ -248,43 +248,45 @@ __global__ __launch_bounds__(THREADS) void topk_regs_kernel(const KvipTopkArgs p
 }
 
 // Split select for rows scored by kvip_hip_indexer_decode (the high-byte histogram is
-// given): the row is cut into segments of 8 keys per thread, one workgroup each, in two
-// launches, so a batch of long rows spreads over many CUs instead of one workgroup per
-// row.
+// given): the row is cut into segments of 2048 or 4096 keys, one 256-thread workgroup each, in two
+// launches, so a batch of long rows spreads over many CUs instead of one workgroup per row.
 //   topk_segment_kernel: every segment workgroup derives the high-byte bin hb from the
 //     row histogram and writes its own low-byte histogram of the keys in hb and its count
 //     of keys above hb.
 //   topk_emit_kernel: every segment workgroup sums those records into the row's kth key
 //     and its own segment prefix (keys > kth and keys == kth in earlier segments), then
 //     emits its segment's selected tokens at their final positions.
-// Both are chains of memory latencies and barriers; the emission also reads every record of its
-// row, so rows above 65536 keys take 8192-key segments of 1024 threads (8 rows of 131072 keys: 16 records
-// of 1 KB per workgroup instead of 64, emission 8.3 -> 6.5 us), and shorter ones 2048-key segments of
-// 256 threads (8 rows of 65536 keys: 10.1 us for both launches against 11.0 with 8192).
 // Record of segment s of a row: words [0, 256) low-byte histogram, [256] keys above hb;
 // segment 0 also holds [257] hb (-1: inconsistent histogram) and [258] keys above hb in
 // the row. The record of a segment is the work-memory record (one per 2048 keys) of its first keys,
 // so that the last word of a row's first record (the fused launch's ticket, select_fetch.hip) is
 // never written.
-constexpr int kSplitKeys = 8;  // keys per thread
+// Both are chains of memory latencies and barriers; the emission also reads every record of its
+// row. Rows above 65536 keys therefore take twice the segment (16 keys per thread), decided by each
+// row's own length, since requests are often far shorter than the stride: 1024-thread workgroups of
+// 8192 keys, chosen by the stride, made 128 rows of 4000 keys 54 % slower (scoring and TopK at stride
+// 131072, 41.9 -> 64.5 us). Scoring and TopK with 2048 keys throughout -> as it is, us: 1 row of 131072
+// keys 23.6 -> 22.0, 8 rows 38.9 -> 37.2, 32 rows 122.8 -> 112.4, 64 rows of 65600-65900 keys 121.8 -> 115.2.
+constexpr int kSplitThreads = 256;
 constexpr int kSegWords = KVIP_TOPK_SEGMENT_WORDS;
-template <int THREADS>
+constexpr int kWideRow = kTopkThreads * 64;  // longer rows take 16 keys per thread
+template <int KPT>
 struct Split {
-    static constexpr int kSegment = THREADS * kSplitKeys;
+    static constexpr int kSegment = kSplitThreads * KPT;
     static constexpr size_t kStep = static_cast<size_t>(kSegment / KVIP_TOPK_SEGMENT_KEYS) * kSegWords;  // words
 };
 
-// Records of row `row`.
+// Records of row `row` (the grid has one workgroup per record).
 KVIP_DEVICE uint32_t* split_records(const KvipTopkArgs& p, int row) {
-    const size_t per_row = (static_cast<size_t>(p.key_stride) + KVIP_TOPK_SEGMENT_KEYS - 1) / KVIP_TOPK_SEGMENT_KEYS;
-    return p.segments + static_cast<size_t>(row) * per_row * kSegWords;
+    return p.segments + static_cast<size_t>(row) * gridDim.x * kSegWords;
 }
 
 KVIP_DEVICE int row_valid(const KvipTopkArgs& p, int row) { return topk_row_valid(p, row); }
 
+template <int KPT>
 KVIP_DEVICE void load_segment(const uint16_t* keys, int first, int stride, uint32_t* kk) {
 #pragma unroll
-    for (int v = 0; v < kSplitKeys / 8; ++v) {
+    for (int v = 0; v < KPT / 8; ++v) {
         const v4i x = *reinterpret_cast<const v4i*>(keys + min(first + v * 8, stride - 8));
         kk[4 * v] = x[0];
         kk[4 * v + 1] = x[1];
@@ -293,28 +295,27 @@ KVIP_DEVICE void load_segment(const uint16_t* keys, int first, int stride, uint3
     }
 }
 
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void topk_segment_kernel(const KvipTopkArgs p) {
+template <int KPT>
+KVIP_DEVICE void split_segment(const KvipTopkArgs& p, int valid) {
     __shared__ uint32_t s_hist[256];
-    __shared__ uint32_t s_wave[THREADS / 64];
+    __shared__ uint32_t s_wave[kSplitThreads / 64];
     __shared__ int s_sel[2];
     const int tid = threadIdx.x;
     const int seg = blockIdx.x;
     const int row = blockIdx.y;
-    const int valid = row_valid(p, row);
-    const int nseg = (valid + Split<THREADS>::kSegment - 1) / Split<THREADS>::kSegment;
+    const int nseg = (valid + Split<KPT>::kSegment - 1) / Split<KPT>::kSegment;
     if (valid < kTopK || seg >= nseg) return;
     int32_t* out = p.topk + static_cast<size_t>(row) * kTopK;
-    uint32_t* rec = split_records(p, row) + seg * Split<THREADS>::kStep;
+    uint32_t* rec = split_records(p, row) + seg * Split<KPT>::kStep;
     // The segment's keys are requested first so that their latency overlaps the bin select.
-    const int first = seg * Split<THREADS>::kSegment + tid * kSplitKeys;
-    const int count = max(0, min(kSplitKeys, valid - first));
-    uint32_t kk[kSplitKeys / 2];
-    load_segment(p.score_keys + static_cast<size_t>(row) * p.key_stride, first, p.key_stride, kk);
+    const int first = seg * Split<KPT>::kSegment + tid * KPT;
+    const int count = max(0, min(KPT, valid - first));
+    uint32_t kk[KPT / 2];
+    load_segment<KPT>(p.score_keys + static_cast<size_t>(row) * p.key_stride, first, p.key_stride, kk);
     // Positions a stale histogram would leave unwritten read -1.
-    for (int i = seg * kTopK / nseg + tid; i < (seg + 1) * kTopK / nseg; i += THREADS) out[i] = -1;
+    for (int i = seg * kTopK / nseg + tid; i < (seg + 1) * kTopK / nseg; i += kSplitThreads) out[i] = -1;
 
-    if (tid < 256) s_hist[tid] = p.histogram[static_cast<size_t>(row) * 256 + tid];
+    s_hist[tid] = p.histogram[static_cast<size_t>(row) * 256 + tid];
     if (tid == 0) s_sel[0] = -1;
     __syncthreads();
     select_bin(s_hist, kTopK, s_sel, s_wave);
@@ -323,11 +324,11 @@ __global__ __launch_bounds__(THREADS) void topk_segment_kernel(const KvipTopkArg
         if (seg == 0 && tid == 0) rec[257] = 0xFFFFFFFFu;
         return;
     }
-    if (tid < 256) s_hist[tid] = 0u;
+    s_hist[tid] = 0u;
     __syncthreads();
     uint32_t above = 0;
 #pragma unroll
-    for (int j = 0; j < kSplitKeys; ++j) {
+    for (int j = 0; j < KPT; ++j) {
         const uint32_t k = (j & 1) ? (kk[j >> 1] >> 16) : (kk[j >> 1] & 0xFFFFu);
         const int high = static_cast<int>(k >> 8);
         if (j < count) {
@@ -337,7 +338,7 @@ __global__ __launch_bounds__(THREADS) void topk_segment_kernel(const KvipTopkArg
     }
     uint32_t total;
     block_exclusive_scan(above, s_wave, &total);  // its barriers also complete the histogram
-    if (tid < 256) rec[tid] = s_hist[tid];
+    rec[tid] = s_hist[tid];
     if (tid == 0) {
         rec[256] = total;
         if (seg == 0) {
@@ -347,66 +348,60 @@ __global__ __launch_bounds__(THREADS) void topk_segment_kernel(const KvipTopkArg
     }
 }
 
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void topk_emit_kernel(const KvipTopkArgs p) {
-    constexpr int kShares = THREADS / 256;  // each bin's records are summed by this many threads
+__global__ __launch_bounds__(kSplitThreads) void topk_segment_kernel(const KvipTopkArgs p) {
+    const int valid = row_valid(p, blockIdx.y);
+    if (valid > kWideRow) split_segment<16>(p, valid);
+    else split_segment<8>(p, valid);
+}
+
+template <int KPT>
+KVIP_DEVICE void split_emit(const KvipTopkArgs& p, int valid) {
     __shared__ uint32_t s_hist[256];
-    __shared__ uint32_t s_all[kShares][256], s_before[kShares][256];
-    __shared__ uint32_t s_wave[THREADS / 64];
+    __shared__ uint32_t s_wave[kSplitThreads / 64];
     __shared__ int s_sel[2];
+    __shared__ uint32_t s_eq_before;
     const int tid = threadIdx.x;
     const int seg = blockIdx.x;
     const int row = blockIdx.y;
-    const int valid = row_valid(p, row);
     int32_t* out = p.topk + static_cast<size_t>(row) * kTopK;
-    if (seg == 0 && tid < 256) p.histogram[static_cast<size_t>(row) * 256 + tid] = 0u;  // ready for the next scoring launch
+    if (seg == 0) p.histogram[static_cast<size_t>(row) * 256 + tid] = 0u;  // ready for the next scoring launch
     if (valid < kTopK) {
         if (seg == 0) {
-            for (int i = tid; i < kTopK; i += THREADS) out[i] = i < valid ? i : -1;
+            for (int i = tid; i < kTopK; i += kSplitThreads) out[i] = i < valid ? i : -1;
         }
         return;
     }
-    const int nseg = (valid + Split<THREADS>::kSegment - 1) / Split<THREADS>::kSegment;
+    const int nseg = (valid + Split<KPT>::kSegment - 1) / Split<KPT>::kSegment;
     if (seg >= nseg) return;
-    const int first = seg * Split<THREADS>::kSegment + tid * kSplitKeys;
-    const int count = max(0, min(kSplitKeys, valid - first));
-    uint32_t kk[kSplitKeys / 2];
-    load_segment(p.score_keys + static_cast<size_t>(row) * p.key_stride, first, p.key_stride, kk);
+    const int first = seg * Split<KPT>::kSegment + tid * KPT;
+    const int count = max(0, min(KPT, valid - first));
+    uint32_t kk[KPT / 2];
+    load_segment<KPT>(p.score_keys + static_cast<size_t>(row) * p.key_stride, first, p.key_stride, kk);
     const uint32_t* recs = split_records(p, row);
-    constexpr size_t kStep = Split<THREADS>::kStep;
+    constexpr size_t kStep = Split<KPT>::kStep;
     const int hb = static_cast<int>(recs[257]);
     if (hb < 0) {
         if (seg == 0 && tid == 0) report(p.status, KVIP_STATUS_HISTOGRAM);
         return;
     }
     const uint32_t gt_hi = recs[258];
-    // Row histogram of the low byte within hb, and this segment's share of earlier counts: thread
-    // (share, bin) sums every kShares-th record, 4 requested per round trip.
-    const int bin = tid & 255, share = tid >> 8;
+    // Row histogram of the low byte within hb, and this segment's share of earlier counts
+    // (KPT records requested per round trip, the last one repeated past the end).
     uint32_t all = 0, before = 0;
-#pragma unroll 4
-    for (int s = share; s < nseg; s += kShares) {
-        const uint32_t c = recs[s * kStep + bin];
-        all += c;
-        before += s < seg ? c : 0u;
+    for (int s0 = 0; s0 < nseg; s0 += KPT) {
+        uint32_t c[KPT];
+#pragma unroll
+        for (int u = 0; u < KPT; ++u) c[u] = recs[min(s0 + u, nseg - 1) * kStep + tid];
+#pragma unroll
+        for (int u = 0; u < KPT; ++u) {
+            all += s0 + u < nseg ? c[u] : 0u;
+            before += s0 + u < seg ? c[u] : 0u;
+        }
     }
     uint32_t above_before = 0;
-    for (int s = tid; s < seg; s += THREADS) above_before += recs[s * kStep + 256];
-    s_all[share][bin] = all;
-    s_before[share][bin] = before;
+    for (int s = tid; s < seg; s += kSplitThreads) above_before += recs[s * kStep + 256];
+    s_hist[tid] = all;
     if (tid == 0) s_sel[0] = -1;
-    __syncthreads();
-    before = 0;
-    if (tid < 256) {
-        all = 0;
-#pragma unroll
-        for (int q = 0; q < kShares; ++q) {
-            all += s_all[q][tid];
-            before += s_before[q][tid];
-        }
-        s_hist[tid] = all;
-        s_before[0][tid] = before;
-    }
     __syncthreads();
     select_bin(s_hist, kTopK - gt_hi, s_sel, s_wave);
     const int lo = s_sel[0];
@@ -417,17 +412,18 @@ __global__ __launch_bounds__(THREADS) void topk_emit_kernel(const KvipTopkArgs p
     const uint32_t kth = (static_cast<uint32_t>(hb) << 8) | static_cast<uint32_t>(lo);
     const uint32_t n_gt = gt_hi + static_cast<uint32_t>(s_sel[1]);
     const uint32_t need = kTopK - n_gt;
+    if (tid == lo) s_eq_before = before;
     uint32_t ngt = 0, neq = 0;
 #pragma unroll
-    for (int j = 0; j < kSplitKeys; ++j) {
+    for (int j = 0; j < KPT; ++j) {
         const uint32_t k = (j & 1) ? (kk[j >> 1] >> 16) : (kk[j >> 1] & 0xFFFFu);
         ngt += (j < count && k > kth) ? 1u : 0u;
         neq += (j < count && k == kth) ? 1u : 0u;
     }
     // Keys above kth in earlier segments, and this segment's prefixes.
     uint32_t gt_before;
-    block_exclusive_scan(above_before + (tid < 256 && tid > lo ? before : 0u), s_wave, &gt_before);
-    const uint32_t eq_before = s_before[0][lo];
+    block_exclusive_scan(above_before + (tid > lo ? before : 0u), s_wave, &gt_before);
+    const uint32_t eq_before = s_eq_before;
     uint32_t total;
     const uint32_t excl = block_exclusive_scan((ngt << 16) | neq, s_wave, &total);
     uint32_t pg = gt_before + (excl >> 16);
@@ -435,7 +431,7 @@ __global__ __launch_bounds__(THREADS) void topk_emit_kernel(const KvipTopkArgs p
     uint32_t err = 0;
     if (ngt != 0u || (neq != 0u && pe < need)) {
 #pragma unroll
-        for (int j = 0; j < kSplitKeys; ++j) {
+        for (int j = 0; j < KPT; ++j) {
             const uint32_t k = (j & 1) ? (kk[j >> 1] >> 16) : (kk[j >> 1] & 0xFFFFu);
             if (j < count) {
                 if (k > kth) {
@@ -452,12 +448,10 @@ __global__ __launch_bounds__(THREADS) void topk_emit_kernel(const KvipTopkArgs p
     report(p.status, err);
 }
 
-template <int THREADS>
-void launch_split(const KvipTopkArgs& a, hipStream_t stream) {
-    const dim3 grid((a.key_stride + Split<THREADS>::kSegment - 1) / Split<THREADS>::kSegment,
-                    a.batch * a.rows_per_request);
-    hipLaunchKernelGGL(topk_segment_kernel<THREADS>, grid, dim3(THREADS), 0, stream, a);
-    hipLaunchKernelGGL(topk_emit_kernel<THREADS>, grid, dim3(THREADS), 0, stream, a);
+__global__ __launch_bounds__(kSplitThreads) void topk_emit_kernel(const KvipTopkArgs p) {
+    const int valid = row_valid(p, blockIdx.y);
+    if (valid > kWideRow) split_emit<16>(p, valid);
+    else split_emit<8>(p, valid);
 }
 
 }  // namespace
@@ -478,7 +472,10 @@ hipError_t launch_topk(const KvipTopkArgs& a, hipStream_t stream) {
     const dim3 grid(a.batch * a.rows_per_request);
     const dim3 block(kTopkThreads);
     if (a.segments != nullptr && a.histogram != nullptr) {
-        a.key_stride > kTopkThreads * 64 ? launch_split<1024>(a, stream) : launch_split<256>(a, stream);
+        const dim3 split((a.key_stride + KVIP_TOPK_SEGMENT_KEYS - 1) / KVIP_TOPK_SEGMENT_KEYS,
+                         a.batch * a.rows_per_request);
+        hipLaunchKernelGGL(topk_segment_kernel, split, dim3(kSplitThreads), 0, stream, a);
+        hipLaunchKernelGGL(topk_emit_kernel, split, dim3(kSplitThreads), 0, stream, a);
         return hipGetLastError();
     }
     // Rows that fit 1024*KPT keys use the register-resident select; a limit (the resident

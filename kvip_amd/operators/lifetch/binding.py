@@ -141,7 +141,7 @@ class LIFetchBinding:
 
     def topk_args(self, use_histogram=True, split=True):
         """TopK arguments; with the scoring histogram a row is selected in 2048-key
-        segments (8192-key ones above 65536 keys) by many workgroups (split=True), or by one
+        segments (4096-key ones above 65536 keys) by many workgroups (split=True), or by one
         workgroup (split=False)."""
         p = abi.ptr
         return abi.TopkArgs(

@@ -475,11 +475,14 @@ def test_forward_of_few_rows_equals_its_stages(torch_gpu, qk, batch, rpr, ctx_lo
     ("few_levels", [100000, 8193]),
     ("all_equal", [70000, 65536, 16384]),
     ("one_bin", [81921, 131071]),
+    ("random", [65536, 65537, 69632, 69633, 70016, 4097, 65535]),
+    ("few_levels", [65544, 65536, 69633]),
 ])
 def test_topk_of_long_rows_on_wide_segments(torch_gpu, kind, ctx):
-    """The split select of rows above 65536 keys (8192-key segments of 1024 threads): rows that end on
-    a segment, one key past it and far before the stride, ties across segments; the work
-    memory's last word of a row's first record stays zero."""
+    """The split select where the stride is above 65536 keys: rows on either side of 65536 (4096-key
+    segments above, 2048-key ones up to it) that end on a segment, one key past it and far before
+    the stride, ties across segments; the work memory's last word of a row's first record stays
+    zero."""
     torch = torch_gpu
     say(f"case wide split {kind} {ctx}")
     rng = np.random.default_rng(len(ctx) * 11 + ctx[0])
