@@ -124,24 +124,38 @@ __global__ __launch_bounds__(PfShape<ELEM>::kThreads, 3 - ELEM) void indexer_pre
     const int n = lane & 31;
     const int g = lane >> 5;
 
+    // Work items (query block, segment), block-fastest: the launch holds one workgroup per
+    // item, or fewer that stride over them (a bounded grid, for callers that run other
+    // kernels beside the prefill: workgroups that run out of items free their CU instead
+    // of queueing more items behind the other kernels).
+    const int nb_items = p.rows / kPfBlockRows + p.sequences;
+    // Block tables are often far wider than the sequences: a workgroup whose first segment starts past
+    // every sequence (its later ones do too) has nothing to do, and leaves before it clears and scans.
+    // The segment is chosen by the table's width: 2 x 1000 rows against 750-1500 keys in tables of 65536
+    // took 34 us with 4096 keys per item, 45 with the shorter one chosen and every workgroup scanning,
+    // 32 as it is (bf16 58, 58 and 37).
+    const int begin = static_cast<int>(blockIdx.x) / nb_items * segment;
+    auto blocks_of = [&](int s) {
+        return s < p.sequences ? max((p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s] + kPfBlockRows - 1) / kPfBlockRows, 0) : 0;
+    };
+    int longest = lane < p.sequences ? p.seq_lens_k[lane] : 0;
+    int mine = blocks_of(tid);
+    asm volatile("" : "+v"(longest), "+v"(mine));  // one memory latency for both
+    for (int s = lane + 64; s - lane < p.sequences; s += 64) longest = max(longest, s < p.sequences ? p.seq_lens_k[s] : 0);
+    if (begin > 0 && __ballot(longest > begin) == 0ull) return;  // uniform
+
     // Query blocks per sequence -> prefix sums; this workgroup's sequence and rows.
     int running = 0;
     for (int base = 0; base < p.sequences; base += kPfThreads) {
         const int s = base + tid;
-        const int c = s < p.sequences ? (p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s] + kPfBlockRows - 1) / kPfBlockRows : 0;
         uint32_t total;
-        const uint32_t excl = block_exclusive_scan(static_cast<uint32_t>(max(c, 0)), s_scan, &total);
+        const uint32_t excl = block_exclusive_scan(static_cast<uint32_t>(base == 0 ? mine : blocks_of(s)), s_scan, &total);
         if (s < p.sequences) s_prefix[s] = running + static_cast<int>(excl);
         running += static_cast<int>(total);
     }
     if (tid == 0) s_prefix[p.sequences] = running;
     for (int i = tid; i < kPfBlockRows * kHistWords; i += kPfThreads) (&s_hist[0][0])[i] = 0u;
     __syncthreads();
-    // Work items (query block, segment), block-fastest: the launch holds one workgroup per
-    // item, or fewer that stride over them (a bounded grid, for callers that run other
-    // kernels beside the prefill: workgroups that run out of items free their CU instead
-    // of queueing more items behind the other kernels).
-    const int nb_items = p.rows / kPfBlockRows + p.sequences;
     const int64_t n_items =
         static_cast<int64_t>(nb_items) * ((p.max_blocks * kBlockTokens + segment - 1) / segment);
     uint32_t err = 0;

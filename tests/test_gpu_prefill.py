@@ -212,3 +212,40 @@ def test_quant_lightning_indexer_wrapper(torch_gpu):
     direct = idx(c["query"], c["weights"], c["query_scale"], c["keys"], c["key_scale"], c["cu"], c["kl"], c["table"])
     assert out.shape == (c["rows"], 1, 2048)
     assert torch.equal(out.view(c["rows"], 2048), direct)
+
+
+@pytest.mark.parametrize("qk", ["fp8", "bf16"])
+@pytest.mark.parametrize("q_lens,k_lens", [
+    ([40], [256]), ([3, 300], [257, 700]), ([2] * 69 + [9], [130] * 69 + [6001]), ([5] * 300, [600] * 150 + [4097] + [600] * 149),
+    ([8], [0])])
+def test_prefill_with_block_tables_wider_than_the_sequences(torch_gpu, qk, q_lens, k_lens):
+    """Tables of 65536 positions against tables of the longest sequence: workgroups whose segment lies
+    past every sequence leave early (the longest is the last of 70 and in the middle of 300
+    sequences here), and keys, visible lengths, histograms and TopK are the same, bit for bit."""
+    torch = torch_gpu
+    say(f"case wide tables {qk} sequences={len(q_lens)} longest={max(k_lens)}")
+    c = make_case(torch, q_lens=q_lens, k_lens=k_lens, heads=64, wdt=torch.float32, qscale=True, kscale=True, seed=23,
+                  qk=qk)
+
+    def run(table, workgroups=0):
+        idx = kvip_amd.PrefillIndexer(torch, max_rows=c["rows"], max_context=max(table.shape[1], 1) * 128,
+                                      max_sequences=len(q_lens), device="cuda")
+        idx.bind(c["query"], c["weights"], c["query_scale"], c["keys"], c["key_scale"], c["cu"], c["kl"], table)
+        idx.score(workgroups)
+        torch.cuda.synchronize()
+        keys, vis, hist = idx.score_keys.clone(), idx.row_valid.clone(), idx.histogram.clone()
+        top = idx.select().clone()
+        assert int(idx.status.item()) == 0
+        return keys, vis, hist, top
+
+    tight = c["table"] if c["table"].shape[1] else torch.zeros((len(q_lens), 1), dtype=torch.int32, device="cuda")
+    wide = torch.zeros((len(q_lens), 512), dtype=torch.int32, device="cuda")
+    wide[:, :tight.shape[1]] = tight
+    want = run(tight)
+    ends = np.concatenate([np.maximum(k - q + 1 + np.arange(q), 0) for q, k in zip(q_lens, k_lens)])
+    assert np.array_equal(want[1].cpu().numpy(), ends)
+    for got in (run(wide), run(wide, 100)):
+        for a, b in zip(got[1:], want[1:]):
+            assert torch.equal(a, b)
+        for r, n in enumerate(ends):
+            assert torch.equal(got[0][r, :n], want[0][r, :n])
