@@ -221,11 +221,6 @@ __global__ __launch_bounds__(kThreads) void lidu_prepare_kernel(const KvipLiduAr
     for (int i = tid; i < kBitmapWords; i += kThreads) {
         s_member[i] = dummy ? 0u : bitmap[i];
     }
-#pragma unroll
-    for (int q = 0; q < kMaxQueries; ++q) {
-        if (q >= qn) continue;
-        for (int i = tid; i < kTileWords / 4; i += kThreads) s_cur[q][i] = make_uint4(0, 0, 0, 0);
-    }
     __syncthreads();
 
     // token_to_slot values from the lookup launch (lidu_lookup_kernel).
@@ -295,6 +290,13 @@ __global__ __launch_bounds__(kThreads) void lidu_prepare_kernel(const KvipLiduAr
             }
         }
     }
+    // Only queries with misses use their bitmap (cleared for every query at the start, a call without
+    // misses took 0.6 us longer).
+#pragma unroll
+    for (int q = 0; q < kMaxQueries; ++q) {
+        if (miss_count[q] == 0) continue;  // uniform
+        for (int i = tid; i < kTileWords / 4; i += kThreads) s_cur[q][i] = make_uint4(0, 0, 0, 0);
+    }
     int status = __syncthreads_or(bad_token) ? kErrTopkToken : kOk;
     stamp(p, profile, b, 1);
 
@@ -326,13 +328,11 @@ __global__ __launch_bounds__(kThreads) void lidu_prepare_kernel(const KvipLiduAr
 #pragma unroll
             for (int q = 0; q < kMaxQueries; ++q) {
                 count[q] = 0;
+                if (miss_count[q] == 0) continue;  // uniform
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    uint4 c = make_uint4(0, 0, 0, 0);
-                    if (miss_count[q] != 0) {
-                        c = s_cur[q][2 * tid + h];
-                        s_cur[q][2 * tid + h] = make_uint4(0, 0, 0, 0);  // for the next tile
-                    }
+                    const uint4 c = s_cur[q][2 * tid + h];
+                    s_cur[q][2 * tid + h] = make_uint4(0, 0, 0, 0);  // for the next tile
                     fresh[q][4 * h + 0] = c.x;
                     fresh[q][4 * h + 1] = c.y;
                     fresh[q][4 * h + 2] = c.z;
@@ -353,6 +353,7 @@ __global__ __launch_bounds__(kThreads) void lidu_prepare_kernel(const KvipLiduAr
                 const uint32_t pres = block_exclusive_scan(count[2 * h] | count[2 * h + 1] << 16, s_wave, &totals);
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
+                    if (miss_count[2 * h + k] == 0) continue;
                     uint32_t o = unique + ((pres >> (16 * k)) & 0xFFFFu);
 #pragma unroll
                     for (int j = 0; j < kTileWordsPerThread; ++j) {

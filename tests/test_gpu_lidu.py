@@ -232,3 +232,19 @@ def test_torch_op_out_variant_in_a_graph_matches_oracle(torch_gpu):
         compare(dev, outs, expect_state, expect, f"op replay{i}")
         for k in lc.STATE:
             case[k] = expect_state[k]
+
+
+@pytest.mark.parametrize("cand", [16384, (1 << 18) + 5000])
+@pytest.mark.parametrize("hitting", [(0, 2), (1, 3), (0, 1, 2), (0, 1, 2, 3)])
+def test_lidu_queries_without_misses_beside_others(torch_gpu, hitting, cand):
+    """Some queries of a request find every token resident (their miss bitmaps are never cleared or
+    read), the others miss, over one and two source tiles; the second request misses throughout."""
+    case = lc.random_case(21, queries=(4, 4), budget=8192, cand=cand, hot_tokens=4096)
+    pool = case["req_pool_entries"][0]
+    slots = case["token_to_slot"][pool, :cand]
+    victim = np.unpackbits(case["miss_slot_bitmap"][0].view(np.uint8), bitorder="little")
+    held = np.flatnonzero((slots >= 0) & (victim[np.maximum(slots, 0)] == 0))
+    rng = np.random.default_rng(len(hitting))
+    for q in hitting:
+        case["topk"][q, 0] = rng.choice(held, ref.SPARSE, replace=False)
+    check_case(torch_gpu, case, f"hitting{hitting} cand={cand}")
