@@ -264,9 +264,10 @@ __global__ __launch_bounds__(THREADS) void topk_regs_kernel(const KvipTopkArgs p
 // Both are chains of memory latencies and barriers; the emission also reads every record of its
 // row. Rows above 65536 keys therefore take twice the segment (16 keys per thread), decided by each
 // row's own length, since requests are often far shorter than the stride: 1024-thread workgroups of
-// 8192 keys, chosen by the stride, made 128 rows of 4000 keys 54 % slower (scoring and TopK at stride
-// 131072, 41.9 -> 64.5 us). Scoring and TopK with 2048 keys throughout -> as it is, us: 1 row of 131072
-// keys 23.6 -> 22.0, 8 rows 38.9 -> 37.2, 32 rows 122.8 -> 112.4, 64 rows of 65600-65900 keys 121.8 -> 115.2.
+// 8192 keys, chosen by the stride, took 26.9 us for 64 rows of 4000 keys at stride 131072, against 16.9
+// with 2048 keys throughout and 9.4 as it is. Both launches, us, 2048 keys throughout -> 8192 -> as it
+// is, stride 131072: 1 row of 131072 keys 11.7, 9.7, 9.5; 8 rows 14.0, 11.2, 11.4; 16 rows 16.5,
+// 11.4, 12.7; 32 rows 26.2, 18.3, 16.3; 64 rows of 8192-32768 18.6, 29.4, 12.4.
 constexpr int kSplitThreads = 256;
 constexpr int kSegWords = KVIP_TOPK_SEGMENT_WORDS;
 constexpr int kWideRow = kTopkThreads * 64;  // longer rows take 16 keys per thread
@@ -276,9 +277,10 @@ struct Split {
     static constexpr size_t kStep = static_cast<size_t>(kSegment / KVIP_TOPK_SEGMENT_KEYS) * kSegWords;  // words
 };
 
-// Records of row `row` (the grid has one workgroup per record).
+// Records of row `row`.
 KVIP_DEVICE uint32_t* split_records(const KvipTopkArgs& p, int row) {
-    return p.segments + static_cast<size_t>(row) * gridDim.x * kSegWords;
+    const size_t per_row = (static_cast<size_t>(p.key_stride) + KVIP_TOPK_SEGMENT_KEYS - 1) / KVIP_TOPK_SEGMENT_KEYS;
+    return p.segments + static_cast<size_t>(row) * per_row * kSegWords;
 }
 
 KVIP_DEVICE int row_valid(const KvipTopkArgs& p, int row) { return topk_row_valid(p, row); }
@@ -380,10 +382,6 @@ KVIP_DEVICE void split_emit(const KvipTopkArgs& p, int valid) {
     const uint32_t* recs = split_records(p, row);
     constexpr size_t kStep = Split<KPT>::kStep;
     const int hb = static_cast<int>(recs[257]);
-    if (hb < 0) {
-        if (seg == 0 && tid == 0) report(p.status, KVIP_STATUS_HISTOGRAM);
-        return;
-    }
     const uint32_t gt_hi = recs[258];
     // Row histogram of the low byte within hb, and this segment's share of earlier counts
     // (KPT records requested per round trip, the last one repeated past the end).
@@ -400,6 +398,10 @@ KVIP_DEVICE void split_emit(const KvipTopkArgs& p, int valid) {
     }
     uint32_t above_before = 0;
     for (int s = tid; s < seg; s += kSplitThreads) above_before += recs[s * kStep + 256];
+    if (hb < 0) {  // stale records; asked here so that their latency passes beside this word's
+        if (seg == 0 && tid == 0) report(p.status, KVIP_STATUS_HISTOGRAM);
+        return;
+    }
     s_hist[tid] = all;
     if (tid == 0) s_sel[0] = -1;
     __syncthreads();
@@ -472,8 +474,11 @@ hipError_t launch_topk(const KvipTopkArgs& a, hipStream_t stream) {
     const dim3 grid(a.batch * a.rows_per_request);
     const dim3 block(kTopkThreads);
     if (a.segments != nullptr && a.histogram != nullptr) {
-        const dim3 split((a.key_stride + KVIP_TOPK_SEGMENT_KEYS - 1) / KVIP_TOPK_SEGMENT_KEYS,
-                         a.batch * a.rows_per_request);
+        // Segments of the longest row of either kind; an odd number, so that the first segments of
+        // consecutive rows, all that short rows have, go to different XCDs (workgroup id % 8).
+        const int wide = (a.key_stride + Split<16>::kSegment - 1) / Split<16>::kSegment;
+        const int narrow = (std::min(a.key_stride, kWideRow) + Split<8>::kSegment - 1) / Split<8>::kSegment;
+        const dim3 split(std::max(wide, narrow) | 1, a.batch * a.rows_per_request);
         hipLaunchKernelGGL(topk_segment_kernel, split, dim3(kSplitThreads), 0, stream, a);
         hipLaunchKernelGGL(topk_emit_kernel, split, dim3(kSplitThreads), 0, stream, a);
         return hipGetLastError();
