@@ -22,12 +22,14 @@
 // half holds half of the heads of the tile's 32 tokens; after the per-lane-half head
 // reduction a v_permlane32_swap adds the other half's heads, and lanes 0-31 scale, round,
 // store the tile's keys and count them. The 256-bin high-byte histogram of the current
-// request is kept per wave in LDS and added to the global row when the wave's range crosses
-// into another request; what the waves of a workgroup hold at the end (mostly one request's) is
-// summed in LDS and added once per workgroup. Adds to one row serialise at ~10 ns each whoever
-// makes them, which bound few long rows when every wave added its own (one row of 32768
-// tokens: 16.2 us, now 7.8; of 131072: 29.0 us, now 11.9). LDS per workgroup stays under 80 KB so that two scoring
-// workgroups leave room on a CU for a 1024-thread TopK workgroup of another row group.
+// request is kept per wave in LDS and added to the global row when a run of its tiles ends. Adds to
+// one row serialise at ~10 ns each whoever makes them, which bound few long rows: where more than 128
+// waves share a request, what the waves of a workgroup hold at the end (mostly one request's) is
+// summed in LDS and added once per workgroup, and no more workgroups than needed take part (one row
+// of 32768 tokens: 16.8 us, now 8.5; of 131072: 30.0, now 12.8). With fewer, holding the adds back and
+// packing the tiles cost more than they save (17 rows of 1500-3000 tokens 6.9 us, 7.5 with both; one
+// of 4096 6.3 and 6.8). LDS per workgroup stays under 80 KB so that two scoring workgroups leave
+// room on a CU for a 1024-thread TopK workgroup of another row group.
 //
 // Reference: QLIMatmul::ComputeMm1 (op_kernel/indexer/indexer_cube.h:161-322),
 // MulWeightAndReduceSum (indexer_score.h:384-426, loop :60-103, finalize :105-140),
@@ -58,8 +60,8 @@ constexpr int kNonTemporal = 2;
 constexpr int kRgLeadWeight = 22;
 constexpr int kRgLagWeight = 18;
 
-// Waves per request above which a workgroup adds its waves' histograms as one (1 us slower at 32
-// waves per row, where the adds are spread; 2 us faster at 256).
+// Waves with tiles per request above which a workgroup adds its waves' histograms as one (1 us slower
+// at 32 waves per row, where the adds are spread; 2 us faster at 256).
 constexpr int kRgCombineWaves = 128;
 
 // Stands in for a missing key-scale array (stride 0): 128 unit scales.
@@ -207,8 +209,11 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     const int64_t nw = static_cast<int64_t>(gridDim.x) * kRgWaves;
     const int64_t w = static_cast<int64_t>(blockIdx.x) * kRgWaves + wave;
     const int64_t weight_total = weight_before(nw);
+    // The waves run independently from here (to the barrier before the last histogram adds when the
+    // workgroup's are combined: with many waves per row; else the barrier costs more than it saves).
+    const bool combine = min(nw, static_cast<int64_t>(total_tiles)) > kRgCombineWaves * p.batch;
     int t, t_end;
-    if (total_tiles <= nw) {  // a tile per wave, packed into the first workgroups (fewer histogram adds)
+    if (combine && total_tiles <= nw) {  // a tile per wave, packed into the first workgroups (fewer histogram adds)
         t = static_cast<int>(w);
         t_end = min(t + 1, total_tiles);
         if (t - wave >= total_tiles) return;  // uniform for the workgroup
@@ -216,9 +221,6 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
         t = static_cast<int>(total_tiles * weight_before(w) / weight_total);
         t_end = static_cast<int>(total_tiles * weight_before(w + 1) / weight_total);
     }
-    // The waves run independently from here (to the barrier before the last histogram adds when the
-    // workgroup's are combined: with many waves per row; else the barrier costs more than it saves).
-    const bool combine = nw > kRgCombineWaves * p.batch;
 
     uint8_t* ring = &s_ring[wave][0][0];
     const uint32_t ring_lds = lds_addr(ring);
@@ -336,8 +338,10 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
             }
             const uint64_t later = run_ends >> i;
             const int run_end = i + static_cast<int>(__builtin_ctzll(later)) + 1;
-            if (held >= 0 && held != b) flush(held);
-            held = b;
+            if (combine) {
+                if (held >= 0 && held != b) flush(held);
+                held = b;
+            }
             for (; i < run_end; ++i) {
                 if (i + 1 < cnt) {
                     issue(i + 1);
@@ -350,11 +354,11 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
                 }
                 score(i);
             }
+            if (!combine) flush(b);
         }
         t += cnt;
     }
     if (!combine) {
-        if (held >= 0) flush(held);
         report(p.status, err);
         return;
     }
@@ -677,8 +681,8 @@ hipError_t launch_ring_kernel(const KvipIndexerArgs& a, int tile_lo, int tile_hi
     auto kernel = indexer_ring_kernel<HEADS, W_BF16>;
     const RingGrid grid = ring_grid(kernel);
     if (grid.blocks == 0) return hipErrorInvalidDevice;
-    // No more workgroups than the block tables have tiles for (one page is one workgroup's four tiles).
-    const int64_t most = static_cast<int64_t>(a.batch) * a.max_blocks;
+    // No more workgroups than the block tables have tiles for (four per page).
+    const int64_t most = static_cast<int64_t>(a.batch) * a.max_blocks * 4;
     const int blocks = static_cast<int>(most < grid.blocks ? most : grid.blocks);
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kRgThreads), 0, stream, a, grid.lead_blocks, tile_lo, tile_hi);
     return hipGetLastError();
