@@ -23,13 +23,14 @@
 // reduction a v_permlane32_swap adds the other half's heads, and lanes 0-31 scale, round,
 // store the tile's keys and count them. The 256-bin high-byte histogram of the current
 // request is kept per wave in LDS and added to the global row when a run of its tiles ends. Adds to
-// one row serialise at ~10 ns each whoever makes them, which bound few long rows: where more than 128
-// waves share a request, what the waves of a workgroup hold at the end (mostly one request's) is
-// summed in LDS and added once per workgroup, and no more workgroups than needed take part (one row
-// of 32768 tokens: 16.8 us, now 8.5; of 131072: 30.0, now 12.8). With fewer, holding the adds back and
-// packing the tiles cost more than they save (17 rows of 1500-3000 tokens 6.9 us, 7.5 with both; one
-// of 4096 6.3 and 6.8). LDS per workgroup stays under 80 KB so that two scoring workgroups leave
-// room on a CU for a 1024-thread TopK workgroup of another row group.
+// one row serialise at ~10 ns each whoever makes them, which bounds launches with a long row: where
+// many waves share the longest request, what the waves of a workgroup hold at the end (mostly one
+// request's) is summed in LDS and added once per workgroup, and few tiles are packed four to a
+// workgroup (one row of 32768 tokens: 16.8 us, now 8.5; of 131072: 30.0, now 12.8; one of 30000 beside
+// 30 of 2000: 16.6, now 10.8). Without such a request, holding the adds back and packing cost more
+// than they save (17 rows of 1500-3000 tokens 6.9 us, 7.5 with both). LDS per workgroup stays
+// under 80 KB so that two scoring workgroups leave room on a CU for a 1024-thread TopK workgroup of
+// another row group.
 //
 // Reference: QLIMatmul::ComputeMm1 (op_kernel/indexer/indexer_cube.h:161-322),
 // MulWeightAndReduceSum (indexer_score.h:384-426, loop :60-103, finalize :105-140),
@@ -60,9 +61,12 @@ constexpr int kNonTemporal = 2;
 constexpr int kRgLeadWeight = 22;
 constexpr int kRgLagWeight = 18;
 
-// Waves with tiles per request above which a workgroup adds its waves' histograms as one (1 us slower
-// at 32 waves per row, where the adds are spread; 2 us faster at 256).
-constexpr int kRgCombineWaves = 128;
+// Waves that share the longest request above which a workgroup adds its waves' histograms as one:
+// where every wave has at most one tile (one row of 2500 tokens, 79 waves, 5.9 us and 6.5 combined;
+// of 4000, 125 waves, 6.5 and 6.2), and where it has several (24 rows of 9000-31000 tokens, up to 131
+// waves, 15.9 and 16.3; 8 rows of 131072, 256 waves, 28.0 either way, and fewer adds beside the TopK).
+constexpr int kRgCombinePacked = 96;
+constexpr int kRgCombineWaves = 160;
 
 // Stands in for a missing key-scale array (stride 0): 128 unit scales.
 __device__ __align__(16) float kRingUnitScale[kBlockTokens] = {
@@ -177,6 +181,7 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     __shared__ int s_prefix[kRgMaxBatch + 1];
     __shared__ uint32_t s_scan[kRgWaves];
     __shared__ int s_req[kRgWaves];  // request of the histogram each wave still holds, -1: none
+    __shared__ int s_long[kRgWaves];  // one of the wave's requests has more than kRgCombinePacked tiles
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -186,16 +191,19 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
 
     // Tile counts per request inside the window [tile_lo, tile_hi) of 32-token tiles ->
     // prefix sums (whole workgroup, before any ring load).
-    int running = 0;
+    int running = 0, longest = 0;
     for (int base = 0; base < p.batch; base += kRgThreads) {
         const int b = base + tid;
         const int c = b < p.batch ? max(0, min((rg_valid(p, b, b) + 31) / 32, tile_hi) - tile_lo) : 0;
+        longest = max(longest, c);
         uint32_t total;
         const uint32_t excl = block_exclusive_scan(static_cast<uint32_t>(c), s_scan, &total);
         if (b < p.batch) s_prefix[b] = running + static_cast<int>(excl);
         running += static_cast<int>(total);
     }
     if (tid == 0) s_prefix[p.batch] = running;
+    const uint64_t some_long = __ballot(longest > kRgCombinePacked);
+    if (lane == 0) s_long[wave] = some_long != 0ull ? 1 : 0;
     for (int i = tid; i < kRgWaves * 256; i += kRgThreads) (&s_hist[0][0])[i] = 0u;
     __syncthreads();
 
@@ -210,8 +218,15 @@ __global__ __launch_bounds__(kRgThreads, 2) void indexer_ring_kernel(const KvipI
     const int64_t w = static_cast<int64_t>(blockIdx.x) * kRgWaves + wave;
     const int64_t weight_total = weight_before(nw);
     // The waves run independently from here (to the barrier before the last histogram adds when the
-    // workgroup's are combined: with many waves per row; else the barrier costs more than it saves).
-    const bool combine = min(nw, static_cast<int64_t>(total_tiles)) > kRgCombineWaves * p.batch;
+    // workgroup's are combined).
+    bool combine = (s_long[0] | s_long[1] | s_long[2] | s_long[3]) != 0;
+    if (combine && total_tiles > nw) {  // several tiles per wave: the waves that share the longest request
+        combine = false;
+        for (int b = lane; b - lane < p.batch && !combine; b += 64) {
+            const int tiles = b < p.batch ? s_prefix[b + 1] - s_prefix[b] : 0;
+            combine = __ballot(tiles * nw > kRgCombineWaves * static_cast<int64_t>(total_tiles)) != 0ull;
+        }
+    }
     int t, t_end;
     if (combine && total_tiles <= nw) {  // a tile per wave, packed into the first workgroups (fewer histogram adds)
         t = static_cast<int>(w);
