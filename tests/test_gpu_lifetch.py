@@ -84,6 +84,37 @@ def test_indexer_scores_match_oracle(torch_gpu, name, qk, heads, wdt, kscale, qs
         assert np.array_equal(hist[r], np.bincount(gpu_keys(rot)[r, :v] >> 8, minlength=256)), r
 
 
+SKEWED_CASES = [
+    # name, ctx: both sides of the lines of the scoring kernel's histogram rule
+    ("one_96_tiles", [3072]),
+    ("one_97_tiles", [3073]),
+    ("long_after_short_packed", [600] * 40 + [12001]),
+    ("long_past_64_requests", [1500] * 64 + [1] * 6 + [30000, 31]),
+    ("equal_12", [6001] * 12),  # 170 of 2048 waves share a request
+    ("equal_13", [6001] * 13),  # 157
+]
+
+
+@pytest.mark.parametrize("name,ctx", SKEWED_CASES, ids=[c[0] for c in SKEWED_CASES])
+def test_indexer_of_skewed_batches_matches_oracle(torch_gpu, name, ctx):
+    """Scores against the oracle, and each row's histogram exactly its keys' own, whether a
+    workgroup adds its waves' histograms as one or each wave its own, with a wave's tiles of one
+    request or of several."""
+    torch = torch_gpu
+    say(f"case skewed {name}")
+    wl = synthetic.decode_workload(torch, batch=len(ctx), ctx=ctx, device="cuda", seed=19)
+    rot, upd, fwd = synthetic.bind(torch, kvip_amd, wl)
+    fwd.score()
+    torch.cuda.synchronize()
+    want, valid = oracle_keys(torch, wl, rot)
+    keys = gpu_keys(rot)
+    assert_scores_close(keys, want, valid, 3e-2)
+    assert int(rot.status.item()) == 0
+    hist = rot.histogram.cpu().numpy()
+    for r, v in enumerate(valid):
+        assert np.array_equal(hist[r], np.bincount(keys[r, :v] >> 8, minlength=256)), r
+
+
 MTP_CASES = [
     # name, rows per request, heads, weight dtype, key scale, query scale, ctx
     ("rows4_h64_fp32w", 4, 64, "f32", True, True, [9000, 4100, 33, 12000, 1, 2049]),
